@@ -441,7 +441,11 @@ typedef struct {
                               fewest keys off their home slots */
 } sp3mm_tuning;
 int sp3mm_get_tuning(sp3mm_tuning *t);
-/* NULL restores the defaults. */
+/* NULL restores the defaults.  While the defaults stand (no schedule set, by
+ * this call, the autotuner or the environment), the FP64 and MIXED64 direct
+ * products, batches and hierarchies adapt the table sizes, group widths and
+ * hash multipliers to a sample of the operands' rows; a schedule that was set
+ * is used as it is. */
 int sp3mm_set_tuning(const sp3mm_tuning *t);
 /* Autotuner: times the direct product R*A*P (opts->precision as in sp3mm_rap)
  * under candidate schedules, `reps` products each, and installs the fastest

@@ -661,6 +661,7 @@ int sp3mm_set_tuning(const sp3mm_tuning *t)
         }
     }
     c->tune = n;
+    c->adapt = !t;
     return 0;
 }
 

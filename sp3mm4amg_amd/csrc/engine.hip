@@ -136,6 +136,8 @@ static void tuning_from_env(Tuning &t)
     if (tuning_valid(e)) t = e;
 }
 
+static bool same_tuning(const Tuning &a, const Tuning &b);
+
 int init_device(int dev)
 {
     std::lock_guard<std::mutex> lk(g_ctx_mu);
@@ -167,6 +169,7 @@ int init_device(int dev)
         if (v >= 16384 && v < c->max_lds) c->max_lds = v;
     }
     tuning_from_env(c->tune);
+    c->adapt = same_tuning(c->tune, Tuning{});
     SP3MM_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
     c->stream = c->own_stream;
     SP3MM_HIP(hipHostMalloc((void **)&c->host_small, 4096, hipHostMallocDefault));
@@ -180,6 +183,12 @@ int init_device(int dev)
         if (c->poll_host) (void)hipHostFree(c->poll_host);
         c->poll_host = nullptr;
         c->poll_dev = nullptr;
+    }
+    if (c->poll_host) {
+        if (hipMalloc((void **)&c->board, sizeof(SampleBoard)) != hipSuccess) {
+            (void)hipGetLastError();
+            c->board = nullptr;
+        }
     }
     // this device's copy of the fixed scratch array (sp3mm_rap_noalloc reports
     // an error if it cannot be resolved; the other entry points do not use it)
@@ -495,7 +504,11 @@ struct Timer {
     }
 };
 
+// the coherent block: the control block at 0, the sample of rows behind it,
+// and the sequence flags of both at its end
 constexpr size_t kPollFlagOff = 4088;
+constexpr size_t kSampleOff = 2048, kSampleFlagOff = 4080;
+static_assert(sizeof(Ctl) <= kSampleOff && kSampleOff + sizeof(SampleOut) <= kSampleFlagOff, "the parts do not overlap");
 
 template <typename Query, typename Block>
 static hipError_t spin_wait(Query q, Block b)
@@ -527,12 +540,11 @@ static int read_ctl(Context *c, const Ctl *d, Ctl &h, Timer *tm = nullptr, int *
 // kPollFlagOff to seq; work queued behind it keeps the GPU busy meanwhile) and
 // copies the block out.  A stream that ends without the flag (a failed launch
 // or a fault) is reported.  seq 0 (no coherent block) reads back with a stream
-// synchronisation instead.
-static int wait_ctl(Context *c, const Ctl *d, unsigned long long seq, Ctl &h)
+// synchronisation instead.  wait_flag waits for any flag of the block.
+static int wait_flag(Context *c, size_t off, unsigned long long seq)
 {
-    if (seq == 0) return read_ctl(c, d, h);
     SP3MM_HIP(hipGetLastError());
-    auto *flag_host = reinterpret_cast<unsigned long long *>(c->poll_host + kPollFlagOff);
+    auto *flag_host = reinterpret_cast<unsigned long long *>(c->poll_host + off);
     for (unsigned spins = 0;; spins++) {
         if (__atomic_load_n(flag_host, __ATOMIC_ACQUIRE) == seq) break;
         if ((spins & 1023) == 1023) {
@@ -549,6 +561,13 @@ static int wait_ctl(Context *c, const Ctl *d, unsigned long long seq, Ctl &h)
         }
         __builtin_ia32_pause();
     }
+    return 0;
+}
+
+static int wait_ctl(Context *c, const Ctl *d, unsigned long long seq, Ctl &h)
+{
+    if (seq == 0) return read_ctl(c, d, h);
+    if (wait_flag(c, kPollFlagOff, seq)) return -1;
     memcpy(&h, c->poll_host, sizeof(Ctl));
     return 0;
 }
@@ -1091,7 +1110,23 @@ static int rap_direct_twopass(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp
 // --------------------------------------------------------------------------
 struct FusedCfg {
     int G, H1, H2;
+    unsigned hm1 = 0, hm2 = 0;  // hash multipliers sampled for the bin (0: the schedule's)
 };
+
+// lanes per row for a stage-1 table of H1 slots
+static int fused_group(const Tuning &tu, int H1) { return H1 <= tu.subwave_h ? 32 : H1 <= 512 ? 64 : 256; }
+
+// The same for sampled tables and a launch of `rows` rows: when the rows do
+// not fill the chip (256 CUs x 24 wavefronts), a row's own latency counts and
+// more lanes share it.  Graph replays, us with 32 / 64 / 256 lanes: 7-point,
+// 128 slots, 1728 rows 47.6 / 44.4 / 54.0, 8000 rows 54.0 / 54.3 / 85.7;
+// second level of a 7-point hierarchy, 512 slots, 1000 rows 135 / 116 / 72,
+// 1728 rows 136 / 98.1 / 97.7, 4096 rows 183 / 140 / 151.
+static int sampled_group(const Tuning &tu, int H1, int64_t rows)
+{
+    const int G = fused_group(tu, H1);
+    return G == 32 && rows <= 6144 ? 64 : H1 > 256 && rows <= 1024 ? 256 : G;
+}
 
 // bins by the upper bound of the R*A row: bin b takes rows with ub <= v_b and
 // runs them with a stage-1 table of H1 = v_b >> h1_shift slots (with shift 0
@@ -1106,7 +1141,7 @@ static void fused_bins(size_t max_lds, bool mixed, const Tuning &tu, BinThreshol
     cfg.clear();
     for (long long v = 64; thr.nb < kMaxBins - 1; v *= 2) {
         const int H1 = (int)std::max<long long>(64, tu.h1_shift >= 0 ? v >> tu.h1_shift : v << -tu.h1_shift);
-        const int G = H1 <= tu.subwave_h ? 32 : H1 <= 512 ? 64 : 256;
+        const int G = fused_group(tu, H1);
         // both tables hold a whole number of group-widths (the compaction and
         // clearing loops step through them G slots at a time)
         const int H2 = std::max(std::max(64, G), H1 / tu.h2_div);
@@ -1115,6 +1150,16 @@ static void fused_bins(size_t max_lds, bool mixed, const Tuning &tu, BinThreshol
         cfg.push_back({G, H1, H2});
     }
     cfg.push_back({0, 0, 0});
+}
+
+// Table slots for rows of at most n distinct keys in the sample: a table at
+// most 3/4 full.  (27-point 100^3 product, 343 keys: 512 slots; a full table
+// sends its row to the long-row kernels, and probing grows past 3/4.)
+static int sampled_slots(int n)
+{
+    int h = kSampleTab;
+    while (3ll * h < 4ll * n) h *= 2;
+    return h;
 }
 
 // The bin the mean row bound nnz(R)/M * nnz(A)/A.M falls in, -1 beyond the
@@ -1159,6 +1204,11 @@ struct FusedPlan {
     // phases, which add gaps to the stream; off unless asked for
     bool detail = false;
     int mk(Timer &tm) const { return detail ? tm.mark() : -1; }
+    // Choose the tables' sizes and multipliers from a sample of R's rows
+    // (large products whose schedule nobody set); sampled: build() did
+    bool adapt = false, sampled = false;
+    bool keep = false;  // the plan will be replayed: sample every bin of it, whatever the product's size
+    int big_from = 0;  // first bin of multi-wavefront groups under the plan's schedule
     // One-off FP64 products may be reassociated: build() stops after the
     // binning and sets `reassoc` when most rows are beyond the one-wavefront
     // tables and the output is wider than an LDS window (the caller then runs
@@ -1213,11 +1263,13 @@ struct FusedPlan {
     int pred = -1;
     Buf pcol, pval, pslotn;
     Buf mlen;             // per-workgroup longest rows of R and A (one-bin test)
+    bool onebin_ok = false;  // the one-bin test is made (decided before the tables are sampled)
     bool onebin = false;  // the binning put every row in bin pred
-    int32_t *slot_col(int i) const { return i == pred ? pcol.as<int32_t>() : scol.as<int32_t>() + soff[i]; }
-    double *slot_val(int i) const { return i == pred ? pval.as<double>() : sval.as<double>() + soff[i]; }
-    int32_t *slot_n(int i) const { return i == pred ? pslotn.as<int32_t>() : slotn.as<int32_t>() + nbase[i]; }
-    int slot_rows(int i) const { return i == pred ? (int)R.M : cnt[i]; }
+    int own = -1;  // the bin launched early (pred, or -1)
+    int32_t *slot_col(int i) const { return i == own ? pcol.as<int32_t>() : scol.as<int32_t>() + soff[i]; }
+    double *slot_val(int i) const { return i == own ? pval.as<double>() : sval.as<double>() + soff[i]; }
+    int32_t *slot_n(int i) const { return i == own ? pslotn.as<int32_t>() : slotn.as<int32_t>() + nbase[i]; }
+    int slot_rows(int i) const { return i == own ? (int)R.M : cnt[i]; }
 
     // The bin whose launch can go ahead of the read-back of the populations:
     // the one the mean row bound nnz(R)/M * nnz(A)/A.M falls in, for FP64
@@ -1236,6 +1288,15 @@ struct FusedPlan {
         const FusedCfg &f = cfg[i];
         const int64_t M = R.M;
         const int *count = early ? &d()->pred_count : d()->counts + i;
+        Tuning t = tu;
+        if (sampled) {
+            // 7-point 128^3 (32-lane groups): u2 = 3 0.412, 2 0.42, 4 0.429 ms;
+            // 27-point 100^3 (wavefronts): u2 = 2 0.442, 3 0.496, 4 0.538 ms
+            t.u2 = f.G == 32 ? 3 : 2;
+            t.slog2_cap = 2;
+            if (f.hm1) t.hash1 = f.hm1;
+            if (f.hm2) t.hash2 = f.hm2;
+        }
         if (mixed)
             launch_direct_mixed(f.G, f.H1, f.H2, slog1, slog2, (float)guard, r(), a(), p(),
                                 lists.as<int32_t>() + (int64_t)i * M, d()->counts + i, cnt[i], rown.as<int32_t>(),
@@ -1245,7 +1306,7 @@ struct FusedPlan {
         else
             launch_direct_fused(f.G, f.H1, f.H2, slog1, slog2, r(), a(), p(), lists.as<int32_t>() + (int64_t)i * M,
                                 count, slot_rows(i), rown.as<int32_t>(), slot_n(i), slot_col(i), slot_val(i),
-                                retry.as<int32_t>(), &d()->nretry, &d()->err, max_blocks(c), s, f32, tu);
+                                retry.as<int32_t>(), &d()->nretry, &d()->err, max_blocks(c), s, f32, t);
     }
 
     // export_ctl: the first gather also copies the control block to the host
@@ -1323,10 +1384,12 @@ struct FusedPlan {
 
     // Bins of at most kMergeRows rows are folded into the next larger non-empty
     // bin while the binning writes its lists (its tables hold their upper
-    // bounds too): a launch of a handful of rows costs a whole row's latency,
-    // while the appended rows fill groups of the larger launch.  d()->counts
-    // holds the merged populations, d()->rawc the populations before.
-    static constexpr int kMergeRows = 1024;
+    // bounds too): a launch that does not fill the chip once (256 CUs x 24
+    // wavefronts) costs a whole row's latency, while the appended rows fill
+    // groups of the larger launch.  27-point 100^3 product: its 3464 boundary
+    // rows took 71 us behind the other 35840 as a launch of their own.
+    // d()->counts holds the merged populations, d()->rawc those before.
+    static constexpr int kMergeRows = 8192;
 
     // The binning clears the control block first; with seq > 0 its scatter
     // kernel also exports the block to the coherent host block with that
@@ -1338,16 +1401,10 @@ struct FusedPlan {
         // rows of R whose columns spread over more than a quarter of A's rows
         // count as unstructured (see wants_reassoc)
         const int span_lim = reassoc_ok ? (int)std::max<int64_t>(1, R.N / 4) : 0;
-        int big_from = thr.nb;
-        for (int i = 0; i < thr.nb; i++)
-            if (cfg[i].G > kWave) {
-                big_from = i;
-                break;
-            }
         // one-bin mode: when the longest row of R times the longest row of A
         // fits the likely bin's bound, every row goes to that bin unmeasured
         OneBin ob{};
-        const bool one = pred >= 0 && cfg[pred].G <= kWave && mlen.p;
+        const bool one = onebin_ok && pred >= 0;
         if (one) {
             ob.part = mlen.as<int>();
             ob.nblk = kMaxLenBlocks;
@@ -1378,21 +1435,130 @@ struct FusedPlan {
     {
         return reassoc_ok && !mixed && !f32 && P.N > (int64_t)window_cap(c->max_lds - 1024);
     }
+    int64_t big = 0;              // rows in multi-wavefront bins and long rows, before bins are merged
     bool wants_reassoc(Context *c) const
     {
         if (mixed || f32) return false;
-        int64_t big = nlong;
-        for (int i = 0; i < thr.nb; i++)
-            if (cfg[i].G > kWave) big += cnt[i];
         return 2 * big >= R.M && 2 * (int64_t)wide >= R.M && R.M > 0 &&
                P.N > (int64_t)window_cap(c->max_lds - 1024);
+    }
+
+    // Sampling costs about 22 us (15 + 6 on the stream, some of it under the
+    // binning's launches), which its tables have to win back.  Host us per
+    // product, sampled / not: 7-point 61x47x53 (4.1e6 stage-1 multiply-adds)
+    // 105 / 85, 57^3 (5.0e6) 111 / 111, 64^3 (7.1e6) 127 / 126, 80^3 (1.4e7)
+    // 173 / 187; 5-point 500^2 (3.7e6) 113 / 92, 700^2 (7.3e6) 146 / 171;
+    // 27-point 36^3 (5.0e6) 120 / 111, 48^3 (1.2e7) 137 / 205.
+    static constexpr double kSampleMacs = 6e6;
+    bool worth_sampling() const { return (double)R.nnz * ((double)A.nnz / (double)A.M) >= kSampleMacs; }
+
+    // Tables, groups and multipliers from the sample: the tables of every bin
+    // that a quarter of the sample fell in hold the most distinct keys seen there (sampled_slots; never more stage-1 slots than
+    // the bin's bound).  Smaller bins take the tables of the next larger such
+    // bin (a few sampled rows miss a bin's maximum: with 256 slots for 27-point
+    // boundary rows of up to 245 keys those 3464 rows ran 275 us), larger ones
+    // keep the bound.  A row
+    // that fills its tables all the same is redone by the long-row kernels,
+    // as under any schedule.  false: nothing usable was sampled.
+    bool apply_sample(Context *c, const SampleOut &so)
+    {
+        std::vector<FusedCfg> f(cfg);
+        int next = -1;
+        for (int b = thr.nb - 1; b >= 0; b--) {
+            const bool known = so.rows[b] > 0 && so.n1[b] < INT32_MAX && so.n2[b] < INT32_MAX;
+            if (known && so.rows[b] >= kSampleRows / 4) {
+                f[b].H1 = std::min((int)thr.v[b], sampled_slots(so.n1[b]));
+                f[b].H2 = sampled_slots(so.n2[b]);
+                next = b;
+            } else if (next >= 0 && (known || so.rows[b] == 0)) {
+                f[b].H1 = std::min((int)thr.v[b], f[next].H1);
+                f[b].H2 = f[next].H2;
+            }
+        }
+        if (next < 0) return false;
+        int64_t slots = 0;
+        for (int b = 0; b < thr.nb; b++) {
+            // small bins fold into larger ones, whose tables must hold their rows
+            if (b > 0) {
+                f[b].H1 = std::max(f[b].H1, f[b - 1].H1);
+                f[b].H2 = std::max(f[b].H2, f[b - 1].H2);
+            }
+            f[b].G = sampled_group(tu, f[b].H1, R.M);
+            f[b].H2 = std::max(std::max(64, f[b].G), f[b].H2);
+            if (fused_lds(f[b].G, f[b].H1, f[b].H2) > c->max_lds) return false;
+            if (so.rows[b] > 0) slots = std::max<int64_t>(slots, f[b].H2);
+        }
+        // scratch slots beyond both the schedule's own and 4 GiB are not worth it
+        if (slots > cfg[pred].H2 && R.M * slots * 12 > ((int64_t)4 << 30)) return false;
+        for (FusedCfg &g : f) take_multipliers(g, so);
+        cfg = f;
+        return true;
+    }
+
+    static void take_multipliers(FusedCfg &f, const SampleOut &so)
+    {
+        f.hm1 = so.cls[0] >= 0 && f.H1 == kSampleTab << so.cls[0] ? so.mul[0] : 0;
+        f.hm2 = so.cls[1] >= 0 && f.H2 == kSampleTab << so.cls[1] ? so.mul[1] : 0;
+    }
+
+    int read_sample(Context *c, unsigned long long seq, SampleOut &so)
+    {
+        if (wait_flag(c, kSampleFlagOff, seq)) return -1;
+        memcpy(&so, c->poll_host + kSampleOff, sizeof so);
+        return 0;
+    }
+
+    unsigned long long queue_sample(Context *c, const int32_t *rows, const int *count, int bin)
+    {
+        const unsigned long long seq = ++c->poll_seq;
+        launch_sample_rows(r(), a(), p(), rows, count, thr, bin, c->board,
+                           reinterpret_cast<SampleOut *>(c->poll_dev + kSampleOff),
+                           reinterpret_cast<unsigned long long *>(c->poll_dev + kSampleFlagOff), seq, c->stream);
+        return seq;
+    }
+
+    // a plan to be replayed: every bin's tables from a sample of its own rows
+    int sample_bins(Context *c)
+    {
+        for (int b = 0; b < thr.nb; b++) {
+            if (cnt[b] == 0) continue;
+            SampleOut so;
+            if (read_sample(c, queue_sample(c, lists.as<int32_t>() + (int64_t)b * R.M, d()->counts + b, -1), so))
+                return -1;
+            int n1 = 0, n2 = 0;  // bins folded into this one report under their own bounds
+            for (int i = 0; i <= thr.nb; i++) {
+                n1 = std::max(n1, so.n1[i]);
+                n2 = std::max(n2, so.n2[i]);
+            }
+            if (n1 == INT32_MAX || n2 == INT32_MAX) continue;
+            FusedCfg f;
+            f.H1 = std::min((int)thr.v[b], sampled_slots(n1));
+            f.G = sampled_group(tu, f.H1, cnt[b]);
+            f.H2 = std::max(std::max(64, f.G), sampled_slots(n2));
+            if (fused_lds(f.G, f.H1, f.H2) > c->max_lds) continue;
+            take_multipliers(f, so);
+            cfg[b] = f;
+            sampled = true;
+        }
+        return 0;
     }
 
     int build(Context *c, Timer &tm)
     {
         hipStream_t s = c->stream;
         const int64_t M = R.M;
+        const bool can_sample = adapt && !mixed && !ext_out && c->board && M > 0;
+        const bool may_sample = can_sample && !keep && worth_sampling();
+        // products too small to sample: wavefronts from 256-slot tables on
+        // (7-point 61x47x53: main kernel 47 -> 38 us) and three left entries
+        // per lane in stage 2
+        if (adapt && !mixed && !keep && !may_sample) {
+            tu.subwave_h = 128;
+            tu.u2 = 3;
+        }
         fused_bins(c->max_lds, mixed, tu, thr, cfg);
+        big_from = 0;
+        while (big_from < thr.nb && cfg[big_from].G <= kWave) big_from++;
         // the binning's buffers first: its kernels start while the rest of
         // the scratch is allocated
         ctl = Buf(sizeof(Ctl));
@@ -1415,11 +1581,14 @@ struct FusedPlan {
         if (pred >= 0) {
             mlen = Buf((size_t)kMaxLenBlocks * 2 * 4);
             if (!mlen.p) (void)hipGetLastError();  // binning measures every row then
+            onebin_ok = mlen.p && cfg[pred].G <= kWave;
         }
         const int e0 = mk(tm);
         // the binning clears the control block, and its scatter kernel sends
         // the populations to the host while the likely bin already runs
         SP3MM_HIP(hipGetLastError());
+        const bool sampling = may_sample && pred >= 0;
+        const unsigned long long sseq = sampling ? queue_sample(c, nullptr, nullptr, pred) : 0;
         const unsigned long long seq = c->poll_host ? ++c->poll_seq : 0;
         launch_binning(c, s, seq);
         const int eu = mk(tm);
@@ -1432,9 +1601,16 @@ struct FusedPlan {
             set_error("scratch allocation failed");
             return -1;
         }
+        // the binning runs while the sample arrives
+        if (sampling) {
+            SampleOut so;
+            if (read_sample(c, sseq, so)) return -1;
+            sampled = apply_sample(c, so);
+        }
         // the likely bin's slots; without them it runs with the other bins
         // after the read-back (its rows are listed like any bin's)
-        if (pred >= 0) {
+        own = can_sample && keep ? -1 : pred;
+        if (own >= 0) {
             const size_t cap = (size_t)M * cfg[pred].H2;
             pcol = Buf(cap * 4);
             pval = Buf(cap * 8);
@@ -1444,13 +1620,13 @@ struct FusedPlan {
                 pcol = Buf();
                 pval = Buf();
                 pslotn = Buf();
-                pred = -1;
+                own = -1;
             }
         }
         int en0 = -1;
-        if (pred >= 0) {
+        if (own >= 0) {
             en0 = mk(tm);
-            launch_main(c, s, pred, true);
+            launch_main(c, s, own, true);
         }
         if (wait_ctl(c, d(), seq, h)) return -1;
         onebin = h.onebin != 0;
@@ -1458,17 +1634,20 @@ struct FusedPlan {
         wide = h.totals[2];
         cnt.assign(h.counts, h.counts + thr.nb + 1);
         nlong = cnt[thr.nb];
+        big = 0;
+        for (int i = big_from; i <= thr.nb; i++) big += h.rawc[i];
         if (reassoc_ok && wants_reassoc(c)) {
             reassoc = true;
             return 0;
         }
+        if (can_sample && keep && sample_bins(c)) return -1;
         soff.assign(thr.nb + 1, 0);
         nbase.assign(thr.nb + 1, 0);
         int64_t ntot = 0, sown = 0;
         stot = 0;
         for (int i = 0; i < thr.nb; i++) {
             stot += (int64_t)cnt[i] * cfg[i].H2;  // slot entries of every row (bounds nnz)
-            if (i == pred) continue;
+            if (i == own) continue;
             soff[i] = sown;
             nbase[i] = ntot;
             sown += (int64_t)cnt[i] * cfg[i].H2;
@@ -1491,7 +1670,7 @@ struct FusedPlan {
         }
         if (en0 < 0) en0 = mk(tm);
         for (int i = 0; i < thr.nb; i++)
-            if (cnt[i] && i != pred) launch_main(c, s, i);
+            if (cnt[i] && i != own) launch_main(c, s, i);
         const int en1 = mk(tm);
         // long and retried rows: count pass of the window kernel (it lists the
         // rows whose windows exceed LDS), then the global dense count for those
@@ -1648,6 +1827,7 @@ static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3m
     plan.rowsum = rowsum;
     plan.reassoc_ok = prec == SP3MM_PREC_FP64 && !rowsum;
     plan.detail = timing;
+    plan.adapt = c->adapt;
     if (plan.build(c, tm)) {
         plan.release_all();
         return -1;
@@ -1678,9 +1858,7 @@ static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3m
             st->nnz_mid = mid;
             st->nnz_out = C.nnz;
             st->main_kernel_launches = 2;
-            st->guarded_entries = plan.nlong;
-            for (int i = 0; i < plan.thr.nb; i++)
-                if (plan.cfg[i].G > kWave) st->guarded_entries += plan.cnt[i];
+            st->guarded_entries = plan.big;
             st->reassociated = 1;
         }
         return 0;
@@ -2278,6 +2456,13 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     reps = std::min(std::max(reps, 1), 50);
     const Tuning saved = c->tune;
+    // candidates are timed as they stand; a schedule the tuner installs stays
+    struct Fixed {
+        Context *c;
+        bool was;
+        ~Fixed() { c->adapt = was; }
+    } fixed{c, c->adapt};
+    c->adapt = false;
     bool reassociated = false;  // the product runs as R*(A*P): the direct kernels' fields do not apply
     // cutoff > 0: a timed product slower than cutoff ends the candidate at
     // once with that time (a schedule whose tables fill and send every row
@@ -2540,6 +2725,7 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
     cur = endb;
     cur_ms = endb_ms;
     c->tune = cur;
+    fixed.was = false;
     best = cur;
     ms_best = cur_ms;
     return 0;
@@ -2573,6 +2759,8 @@ static int batch_build(Context *c, Batch *b, bool graph)
     b->plan.mixed = b->prec == SP3MM_PREC_MIXED;
     b->plan.f32 = b->mixed;
     b->plan.tu = c->tune;
+    b->plan.adapt = c->adapt;
+    b->plan.keep = true;
     b->plan.guard = b->guard;
     if (b->plan.build(c, tm)) return -1;
     const int e2 = tm.mark();
@@ -2772,6 +2960,46 @@ int batch_repack(void *h, int count, const sp3mm_dmat *R, const sp3mm_dmat *A, c
     return 0;
 }
 
+// A replay saw other sizes than its plan's.  Under sampled tables that can be
+// a pattern of the same sizes whose rows have more distinct keys than the
+// sampled ones: such a batch is rebuilt with bound-sized tables and goes on.
+// Any other change of size stays refused (-1, the error as it was set).
+static int batch_refit(Context *c, Batch *b)
+{
+    char why[600];
+    snprintf(why, sizeof why, "%s", last_error_text());
+    FusedPlan old = std::move(b->plan);
+    b->plan = FusedPlan();
+    const bool graph = b->exec != nullptr;
+    const hipGraph_t g = b->graph;
+    const hipGraphExec_t x = b->exec;
+    b->graph = nullptr;
+    b->exec = nullptr;
+    const bool adapt = c->adapt;
+    const Tuning tune = c->tune;
+    c->adapt = false;
+    c->tune = old.tu;
+    const int rc = batch_build(c, b, graph);
+    c->adapt = adapt;
+    c->tune = tune;
+    if (rc == 0 && b->plan.nnz == old.nnz && b->plan.cnt == old.cnt && b->plan.nretry == 0 &&
+        b->plan.nspill == old.nspill && (b->exec != nullptr) == graph) {
+        if (x) (void)hipGraphExecDestroy(x);
+        if (g) (void)hipGraphDestroy(g);
+        old.release_all();
+        return 0;
+    }
+    (void)hipStreamSynchronize(c->stream);
+    if (b->exec) (void)hipGraphExecDestroy(b->exec);
+    if (b->graph) (void)hipGraphDestroy(b->graph);
+    b->plan.release_all();
+    b->plan = std::move(old);
+    b->graph = g;
+    b->exec = x;
+    set_error("%s", why);
+    return -1;
+}
+
 int batch_run(void *h, bool use_graph, double *ms)
 {
     Context *c = ctx();
@@ -2795,6 +3023,7 @@ int batch_run(void *h, bool use_graph, double *ms)
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (ms) *ms = t;
+    if (rc && b->plan.sampled && batch_refit(c, b) == 0) return batch_run(h, use_graph, ms);
     return rc;
 }
 
@@ -2999,6 +3228,8 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
         L.rap.A = cur;
         L.rap.P = L.pplan.C;
         L.rap.tu = c->tune;
+        L.rap.adapt = c->adapt;
+        L.rap.keep = true;
         if (L.rap.build(c, t2)) {
             hier_release(h);
             return nullptr;

@@ -53,6 +53,10 @@ struct Context {
     Pool pool;
     // scheduling of the one-pass direct kernels (sp3mm_set_tuning / sp3mm_autotune)
     Tuning tune;
+    // no schedule was set: large products take their table sizes and hash
+    // multipliers from a sample of their rows (FusedPlan::adapt)
+    bool adapt = true;
+    SampleBoard *board = nullptr;  // device scratch of the sampling (null: not available)
     // device address of the fixed scratch array of the allocation-free entry
     // point on this device (null if it could not be resolved)
     unsigned char *noalloc_base = nullptr;

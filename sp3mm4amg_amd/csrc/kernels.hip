@@ -412,7 +412,7 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_scatter(const int64_t *__re
             bool reassoc = false;
             if (ex.reassoc_possible) {
                 long long big = 0;
-                for (int b = ex.big_from; b < nbin; b++) big += merge_lim > 0 ? cnt[b] : raw[b];
+                for (int b = ex.big_from; b < nbin; b++) big += raw[b];
                 reassoc = 2 * big >= M && 2 * (long long)ex.totals[2] >= M;
             }
             *ex.pred_count = reassoc || ex.pred < 0 ? 0 : (merge_lim > 0 ? cnt[ex.pred] : raw[ex.pred]);
@@ -1003,6 +1003,283 @@ __global__ void __launch_bounds__(256) k_hash_score(SpOperand R, SpOperand A, Sp
         }
         wave_sync();
     }
+}
+
+// ---------------------------------------------------------------------------
+// table sizes and hash multipliers of one product, from a sample of its rows
+// ---------------------------------------------------------------------------
+// A product whose schedule nobody fixed takes its table sizes and multipliers
+// from its own operands: kSampleRows rows of R, one per equal part of the rows
+// at a pseudo-random place in it (evenly spaced rows of a mesh can all lie on
+// a boundary).  A workgroup collects its row's distinct stage-1 keys (eight
+// lanes walk a row of A) and stage-2 keys (four lanes a row of P) through
+// dedup tables, appending every new key to a list; kSampleSplit workgroups
+// take the same row and a share of the candidates each.  A wavefront scores a
+// candidate by the probes linear probing would make: it counts the keys per
+// home slot, and the keys a slot passes on to the next one follow from the
+// counts alone, carry' = max(0, carry + count - 1), composed over the lanes as
+// maps x -> max(a, x + b); their sum is the keys' total distance from home.
+// k_sample_pick (one workgroup) then adds the rows' scores up and writes the
+// choice to coherent host memory.  Sums and maxima go through plain stores
+// and the kernel boundary: atomics of 256 workgroups on a few lines took 50 us.
+constexpr int kSampThreads = 512;
+constexpr int kSampTab1 = 4096, kSampTab2 = 2048;  // dedup tables; lists of half as many keys
+constexpr int kSampProbes = 64;                    // probes after which a dedup table counts as full
+
+// candidate multiplier i: 2^32/phi first, then odd numbers of a fixed splitmix64 list
+__device__ __forceinline__ unsigned sample_mul(int i)
+{
+    if (i == 0) return kHashMul;
+    uint64_t z = 0x9E3779B97F4A7C15ull * (uint64_t)(i + 1);
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return (unsigned)(z >> 32) | 1u;
+}
+
+// appends `key` to list (at most cap keys) when the dedup table did not hold
+// it; *over: the table or the list is full
+__device__ __forceinline__ void sample_insert(int *tab, int logtab, int *list, int cap, int *n, int *over, int key)
+{
+    const unsigned mask = (1u << logtab) - 1;
+    unsigned s = hslot(key, 32 - logtab);
+    for (int probe = 0; probe < kSampProbes; probe++) {
+        const int old = atomicCAS(tab + s, kEmpty, key);
+        if (old == key) return;
+        if (old == kEmpty) {
+            const int at = atomicAdd(n, 1);
+            if (at < cap) list[at] = key;
+            else *over = 1;
+            return;
+        }
+        s = (s + 1) & mask;
+    }
+    *over = 1;
+}
+
+// table class of n keys: at most 3/4 full (the host's sampled_slots)
+__device__ __forceinline__ int sample_class(int n)
+{
+    int cls = 0;
+    while (cls < kSampleClasses && 3ll * (kSampleTab << cls) < 4ll * n) cls++;
+    return cls < kSampleClasses ? cls : -1;
+}
+
+// x -> max(a, x + b), the carry past a run of slots
+struct CarryMap {
+    int a, b;
+};
+__device__ __forceinline__ CarryMap then(CarryMap f, CarryMap g) { return {max(g.a, f.a + g.b), f.b + g.b}; }
+
+// summed distance from home of n distinct keys in a table of kWave * E slots
+// (linear probing, circular); `cntt` holds that many ints
+template <int E>
+__device__ __forceinline__ int sample_distance(const int *key, int n, int sh, unsigned mul, int *cntt, int l)
+{
+#pragma unroll
+    for (int j = 0; j < E; j++) cntt[j * kWave + l] = 0;
+    wave_sync();
+    for (int i = l; i < n; i += kWave) atomicAdd(cntt + hslot(key[i], sh, mul), 1);
+    wave_sync();
+    int h[E];
+    CarryMap m{0, 0};
+#pragma unroll
+    for (int j = 0; j < E; j++) {  // this lane's E consecutive slots
+        h[j] = cntt[l * E + j];
+        m = then(m, CarryMap{0, h[j] - 1});
+    }
+    // inclusive composition over the lanes
+    for (int o = 1; o < kWave; o <<= 1) {
+        CarryMap p{__shfl_up(m.a, o), __shfl_up(m.b, o)};
+        if (l >= o) m = then(p, m);
+    }
+    // the carry around the end is what the whole table passes on from an
+    // empty start (once around settles it: the table is not full)
+    const int wrap = max(0, __shfl(m.a, kWave - 1));
+    CarryMap before{__shfl_up(m.a, 1), __shfl_up(m.b, 1)};
+    int x = l == 0 ? wrap : max(before.a, wrap + before.b);
+    int sum = 0;
+#pragma unroll
+    for (int j = 0; j < E; j++) {
+        x = max(0, x + h[j] - 1);
+        sum += x;
+    }
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o);
+    return sum;
+}
+
+__global__ void __launch_bounds__(kSampThreads) k_sample_rows(SpOperand R, SpOperand A, SpOperand P,
+                                                             const int32_t *__restrict__ rows,
+                                                             const int *__restrict__ count, BinThresholds thr,
+                                                             SampleBoard *__restrict__ board)
+{
+    __shared__ int d1[kSampTab1], d2[kSampTab2], l1[kSampTab1 / 2], l2[kSampTab2 / 2];
+    constexpr int kScoreH = kSampleTab << (kSampleClasses - 1);
+    constexpr int kSampWaves = kSampThreads / kWave;
+    __shared__ int tabs[kSampWaves][kScoreH];
+    __shared__ int cnt[2], over;
+    __shared__ unsigned long long ubsh;
+    const int t = threadIdx.x, w = t / kWave, l = t % kWave;
+    for (int i = t; i < kSampTab1; i += kSampThreads) d1[i] = kEmpty;
+    for (int i = t; i < kSampTab2; i += kSampThreads) d2[i] = kEmpty;
+    if (t == 0) {
+        cnt[0] = cnt[1] = 0;
+        over = 0;
+        ubsh = 0;
+    }
+    __syncthreads();
+    const int part = blockIdx.x / kSampleSplit, share = blockIdx.x % kSampleSplit;
+    // row `part` of the sample: a place in [part, part + 1) * M / kSampleRows
+    const int64_t M = rows ? *count : R.M;
+    const int64_t lo = part * M / kSampleRows, hi = (part + 1) * M / kSampleRows;
+    const int64_t at = min(lo + (int64_t)(((uint64_t)sample_mul(part + 1) * (uint64_t)max((int64_t)1, hi - lo)) >> 32),
+                           M - 1);
+    const int64_t r = rows ? rows[at] : at;
+    const int64_t rb = R.rp[r], re = R.rp[r + 1];
+    unsigned long long u = 0;
+    for (int64_t e = rb + (t >> 3); e < re; e += kSampThreads / 8) {
+        const int k = R.col[e];
+        const int q0 = A.rp32[k], q1 = A.rp32[k + 1];
+        if ((t & 7) == 0) u += (unsigned)(q1 - q0);
+        for (int q = q0 + (t & 7); q < q1 && !over; q += 8)
+            sample_insert(d1, 12, l1, kSampTab1 / 2, cnt, &over, A.col[q]);
+    }
+    if (u) atomicAdd(&ubsh, u);
+    __syncthreads();
+    const bool full1 = over != 0;
+    const int n1 = min(cnt[0], kSampTab1 / 2);
+    __syncthreads();
+    if (!full1)
+        for (int i = t >> 2; i < n1; i += kSampThreads / 4) {
+            const int k = l1[i];
+            const int q1 = P.rp32[k + 1];
+            for (int q = P.rp32[k] + (t & 3); q < q1 && !over; q += 4)
+                sample_insert(d2, 11, l2, kSampTab2 / 2, cnt + 1, &over, P.col[q]);
+        }
+    __syncthreads();
+    const bool full2 = over != 0;
+    const int n2 = min(cnt[1], kSampTab2 / 2);
+    if (t == 0 && share == 0) {
+        int b = 0;
+        while (b < thr.nb && (long long)ubsh > thr.v[b]) b++;
+        board->bin[part] = ubsh > 0 ? b : -1;
+        board->n[0][part] = full1 ? INT32_MAX : n1;
+        board->n[1][part] = full2 ? INT32_MAX : n2;
+    }
+    for (int st = 0; st < 2; st++) {
+        const int n = st ? n2 : n1;
+        const int *key = st ? l2 : l1;
+        const int cls = (st ? full2 : full1) ? -1 : sample_class(n);
+        if (cls < 0) continue;
+        const int sh = 32 - 6 - cls;
+        static_assert(kSampleTab == 64 && kSampleClasses == 5, "the shift above, the cases below");
+        int *tab = tabs[w];
+        for (int c = share + kSampleSplit * w; c < kSampleCand; c += kSampleSplit * kSampWaves) {
+            const unsigned mul = sample_mul(c);
+            int d;
+            switch (cls) {
+            case 0: d = sample_distance<1>(key, n, sh, mul, tab, l); break;
+            case 1: d = sample_distance<2>(key, n, sh, mul, tab, l); break;
+            case 2: d = sample_distance<4>(key, n, sh, mul, tab, l); break;
+            case 3: d = sample_distance<8>(key, n, sh, mul, tab, l); break;
+            default: d = sample_distance<16>(key, n, sh, mul, tab, l); break;
+            }
+            if (l == 0) board->score[part][st][c] = (unsigned short)min(d, 0xFFFF);
+        }
+    }
+}
+
+// one workgroup: per-bin maxima, and per stage the candidate with the smallest
+// sum over the rows whose keys take the likely bin's table
+constexpr int kPickThreads = 1024;
+__global__ void __launch_bounds__(kPickThreads) k_sample_pick(const SampleBoard *__restrict__ board, int pred,
+                                                             SampleOut *host, unsigned long long *flag,
+                                                             unsigned long long seq)
+{
+    __shared__ int rows[kMaxBins + 1], n1[kMaxBins + 1], n2[kMaxBins + 1], rcls[2][kSampleRows];
+    __shared__ unsigned sum[2 * kSampleCand];
+    __shared__ int tops[2];
+    const int t = threadIdx.x;
+    if (t < 2 * kSampleCand) sum[t] = 0;
+    if (t <= kMaxBins) rows[t] = n1[t] = n2[t] = 0;
+    __syncthreads();
+    if (t < kSampleRows) {
+        const int b = board->bin[t], a1 = board->n[0][t], a2 = board->n[1][t];
+        if (b >= 0) {
+            atomicAdd(rows + b, 1);
+            atomicMax(n1 + b, a1);
+            atomicMax(n2 + b, a2);
+        }
+        rcls[0][t] = a1 < INT32_MAX ? sample_class(a1) : -1;
+        rcls[1][t] = a2 < INT32_MAX ? sample_class(a2) : -1;
+    }
+    __syncthreads();
+    // the tables to score for: those of the rows of bin `pred` (-1: of all)
+    if (t < 2) {
+        const int *n = t ? n2 : n1;
+        int m = pred >= 0 ? n[pred] : 0;
+        for (int b = 0; pred < 0 && b <= kMaxBins; b++) m = max(m, n[b]);
+        tops[t] = m;
+    }
+    __syncthreads();
+    // eight scores per load, all of a thread's loads in flight together
+    constexpr int kChunks = 2 * kSampleCand / 8;  // of one row
+    constexpr int kRowsAt = kPickThreads / kChunks;
+    static_assert(kSampleRows % kRowsAt == 0, "whole rows per step");
+    const int ch = t % kChunks, st = ch / (kSampleCand / 8);
+    const int cls = tops[st] < INT32_MAX ? sample_class(tops[st]) : -1;
+    uint4 raw[kSampleRows / kRowsAt];
+#pragma unroll
+    for (int i = 0; i < kSampleRows / kRowsAt; i++)
+        raw[i] = reinterpret_cast<const uint4 *>(board->score[i * kRowsAt + t / kChunks])[ch];
+    unsigned s[8] = {};
+#pragma unroll
+    for (int i = 0; i < kSampleRows / kRowsAt; i++) {
+        // a row of another class wrote no scores for this table
+        const bool use = cls >= 0 && rcls[st][i * kRowsAt + t / kChunks] == cls;
+        const unsigned x[4] = {raw[i].x, raw[i].y, raw[i].z, raw[i].w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            s[2 * j] += use ? x[j] & 0xFFFFu : 0u;
+            s[2 * j + 1] += use ? x[j] >> 16 : 0u;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+        if (s[j]) atomicAdd(sum + ch * 8 + j, s[j]);
+    __syncthreads();
+    // smallest sum, the earliest candidate of equals: one wavefront per stage
+    if (t < 2 * kWave) {
+        const int ps = t / kWave;
+        unsigned v = 0xFFFFFFFFu;
+        for (int c = t % kWave; c < kSampleCand; c += kWave)
+            v = min(v, min(sum[ps * kSampleCand + c], 0xFFFFFEu) << 8 | (unsigned)c);
+        for (int o = 32; o > 0; o >>= 1) v = min(v, (unsigned)__shfl_xor((int)v, o));
+        const int ptop = tops[ps];
+        if (t % kWave == 0) {
+            __hip_atomic_store(&host->cls[ps], ptop < INT32_MAX ? sample_class(ptop) : -1, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+            __hip_atomic_store(&host->mul[ps], sample_mul((int)(v & 255u)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
+    if (t <= kMaxBins) {
+        __hip_atomic_store(&host->rows[t], rows[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&host->n1[t], n1[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __hip_atomic_store(&host->n2[t], n2[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __threadfence_system();
+    __syncthreads();
+    if (t == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+void launch_sample_rows(const SpOperand &R, const SpOperand &A, const SpOperand &P, const int32_t *rows,
+                        const int *count, const BinThresholds &thr, int pred,
+                        SampleBoard *board, SampleOut *host, unsigned long long *flag, unsigned long long seq,
+                        hipStream_t st)
+{
+    hipLaunchKernelGGL(k_sample_rows, dim3(kSampleRows * kSampleSplit), dim3(kSampThreads), 0, st, R, A, P, rows,
+                       count, thr, board);
+    hipLaunchKernelGGL(k_sample_pick, dim3(1), dim3(kPickThreads), 0, st, board, pred, host, flag, seq);
 }
 
 // ---------------------------------------------------------------------------

@@ -148,6 +148,33 @@ void launch_direct_fused(int G, int H1, int H2, int slog1, int slog2, const SpOp
                          int32_t *rownnz, int32_t *slotn, int32_t *scol, double *sval, int32_t *retry,
                          int *nretry, int *err, int max_blocks, hipStream_t st, bool f32in,
                          const Tuning &tu);
+// What k_sample_rows learns from kSampleRows rows of R: per bin of the row
+// bound the number of rows sampled and the most distinct stage-1 and stage-2
+// keys of any of them (INT32_MAX: more than the kernel counts), and per stage
+// the hash multiplier whose tables of kSampleTab << cls slots need the fewest
+// probes for the sampled rows with that many keys (cls: the table for the
+// row with the most keys in bin `pred`, or of all for pred < 0; -1: none scored).
+constexpr int kSampleRows = 64;
+constexpr int kSampleSplit = 8;    // workgroups per sampled row (a share of the candidates each)
+constexpr int kSampleTab = 64;
+constexpr int kSampleClasses = 5;  // tables of 64 .. 1024 slots are scored
+constexpr int kSampleCand = 256;
+struct SampleOut {
+    int rows[kMaxBins + 1], n1[kMaxBins + 1], n2[kMaxBins + 1];
+    int cls[2];
+    unsigned mul[2];
+};
+// device scratch of the sampling: a sampled row's bin and key counts, and its
+// score of every candidate
+struct SampleBoard {
+    int bin[kSampleRows], n[2][kSampleRows];
+    alignas(16) unsigned short score[kSampleRows][2][kSampleCand];
+};
+// rows / count (device): sample a list of rows instead of all of R's
+void launch_sample_rows(const SpOperand &R, const SpOperand &A, const SpOperand &P, const int32_t *rows,
+                        const int *count, const BinThresholds &thr, int pred,
+                        SampleBoard *board, SampleOut *host, unsigned long long *flag, unsigned long long seq,
+                        hipStream_t st);
 // Scores of candidate hash multipliers for the direct kernel's tables of H1 and
 // H2 slots (both at most kScoreTable) on sample rows of R (see k_hash_score):
 // score1[c] / score2[c] (zeroed here) receive the summed home-slot distances,
