@@ -238,7 +238,8 @@ typedef struct {
                                 (long rows and rows whose tables filled)       */
     int32_t main_kernel_launches;
     int32_t spilled_rows;  /* direct path: of those, rows whose column windows
-                              exceeded LDS (global dense accumulators)          */
+                              exceeded LDS (global dense accumulators, or
+                              products forwarded without summing R*A first)     */
     int32_t reassociated;  /* direct path: 1 if the product ran as R*(A*P)
                               (most rows beyond the one-wavefront tables and
                               an output wider than an LDS window)               */

@@ -6,6 +6,7 @@
 // populations, then output size) to size grids and the output arrays.
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 #include <cstdarg>
 #include <cstdlib>
 #include <cstdio>
@@ -401,7 +402,7 @@ struct Ctl {
     int nretry;
     int err;
     int nspill;  // long rows whose column windows exceed the LDS window kernel
-    int pad;
+    int nwide;   // rows of k_scatter_direct whose windows would
     unsigned long long totals[3];  // bound sum, bound maximum, rows of unstructured spread
     int64_t nnz;
     int64_t pad2;
@@ -1111,6 +1112,7 @@ static int rap_direct_twopass(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp
 struct FusedCfg {
     int G, H1, H2;
     unsigned hm1 = 0, hm2 = 0;  // hash multipliers sampled for the bin (0: the schedule's)
+    bool scatter = false;       // run by k_scatter_direct, in slots of H2 entries
 };
 
 // lanes per row for a stage-1 table of H1 slots
@@ -1188,7 +1190,7 @@ struct FusedPlan {
     std::vector<FusedCfg> cfg;
     std::vector<int> cnt, fcnt;
     std::vector<int64_t> soff, nbase;
-    int nlong = 0, nretry = 0, nspill = 0;
+    int nlong = 0, nretry = 0, nspill = 0, nwide = 0;
     bool built = false;  // build() has read the retry and spill counts
     bool spec = false;   // tail launched before the retry count is known
     // the speculative tail leaves rows whose tables filled for later: their
@@ -1248,6 +1250,7 @@ struct FusedPlan {
     Buf lslotn, lcol, lval;
     int lcap = 0;
     bool lslots = false;
+    bool lscatter = false;  // the long rows are run by k_scatter_direct
     DenseDirectWs sws;  // global dense workspace of the spilled rows
     sp3mm_dmat C{};
     double ms_ub = 0, ms_num = 0, ms_scan = 0;
@@ -1297,7 +1300,11 @@ struct FusedPlan {
             if (f.hm1) t.hash1 = f.hm1;
             if (f.hm2) t.hash2 = f.hm2;
         }
-        if (mixed)
+        if (f.scatter)
+            launch_scatter_direct(c->num_cu, r(), a(), p(), lists.as<int32_t>() + (int64_t)i * M, count, slot_rows(i),
+                                  f.H2, rown.as<int32_t>(), slot_n(i), slot_col(i), slot_val(i),
+                                  window_cap(c->max_lds - 1024), &d()->nwide, &d()->err, s, f32);
+        else if (mixed)
             launch_direct_mixed(f.G, f.H1, f.H2, slog1, slog2, (float)guard, r(), a(), p(),
                                 lists.as<int32_t>() + (int64_t)i * M, d()->counts + i, cnt[i], rown.as<int32_t>(),
                                 slotn.as<int32_t>() + nbase[i], scol.as<int32_t>() + soff[i],
@@ -1344,7 +1351,11 @@ struct FusedPlan {
         int32_t *llist = lists.as<int32_t>() + (int64_t)thr.nb * M;
         if (nlong > 0 && lslots) {
             // one pass into the slots at count time, a gather in the tail
-            if (!num)
+            if (!num && lscatter)
+                launch_scatter_direct(c->num_cu, r(), a(), p(), llist, d()->counts + thr.nb, nlong, lcap,
+                                      rown.as<int32_t>(), lslotn.as<int32_t>(), lcol.as<int32_t>(), lval.as<double>(),
+                                      window_cap(c->max_lds - 1024), &d()->nwide, &d()->err, s, f32);
+            else if (!num)
                 launch_window_direct(true, std::min(nlong, c->num_cu), wl, r(), a(), p(), llist,
                                      d()->counts + thr.nb, dlog1, spill.as<int32_t>(), &d()->nspill,
                                      rown.as<int32_t>(), nullptr, nullptr, nullptr, mixed ? rowsum : nullptr, 0,
@@ -1449,8 +1460,16 @@ struct FusedPlan {
     // 105 / 85, 57^3 (5.0e6) 111 / 111, 64^3 (7.1e6) 127 / 126, 80^3 (1.4e7)
     // 173 / 187; 5-point 500^2 (3.7e6) 113 / 92, 700^2 (7.3e6) 146 / 171;
     // 27-point 36^3 (5.0e6) 120 / 111, 48^3 (1.2e7) 137 / 205.
-    static constexpr double kSampleMacs = 6e6;
-    bool worth_sampling() const { return (double)R.nnz * ((double)A.nnz / (double)A.M) >= kSampleMacs; }
+    // Few stage-1 products can still forward into long rows of P: 4,000-row
+    // lognormal operator (1.6e6, rows of P of 20), 0.97 ms unsampled and 0.57
+    // with the sample, which finds the rows unstructured (wants_scatter).
+    static constexpr double kSampleMacs = 6e6, kSampleLongP = 8, kSampleForward = 2.5e7;
+    bool worth_sampling() const
+    {
+        const double macs = (double)R.nnz * ((double)A.nnz / (double)A.M);
+        const double lp = (double)P.nnz / (double)std::max<int64_t>(1, P.M);
+        return macs >= kSampleMacs || (lp >= kSampleLongP && macs * lp >= kSampleForward);
+    }
 
     // Tables, groups and multipliers from the sample: the tables of every bin
     // that a quarter of the sample fell in hold the most distinct keys seen there (sampled_slots; never more stage-1 slots than
@@ -1493,6 +1512,52 @@ struct FusedPlan {
         for (FusedCfg &g : f) take_multipliers(g, so);
         cfg = f;
         return true;
+    }
+
+    // Forwarding without merging (k_scatter_direct) for the rows of
+    // multi-wavefront bins and the long rows: when at least half of the sampled
+    // rows are such rows, at least half spread their columns over more than a
+    // quarter of A's rows, merging R*A would leave more than a quarter of
+    // the forwarded products, P's columns fit the LDS accumulators (wider outputs are
+    // reassociated, see wants_reassoc) and the slots fit 4 GiB.  Lognormal
+    // operators of 4,000 / 10,000 / 60,000 rows: 0.97 / 3.45 / 40.4 ms when
+    // their rows filled the hash tables and went to the dense long-row
+    // kernels, 0.57 / 0.81 / 4.0 ms here.
+    static constexpr double kScatterMerge = 4.0;
+    int scatter_slots() const { return (int)((P.N + 31) / 32 * 32); }
+    bool wants_scatter(Context *c, const SampleOut &so) const
+    {
+        int rows = 0, bigrows = 0, wide = 0;
+        int64_t prods = 0, keys = 0, bound = 0;
+        for (int b = 0; b <= thr.nb; b++) {
+            rows += so.rows[b];
+            wide += so.wide[b];
+            if (b < big_from) continue;
+            bigrows += so.rows[b];
+            prods += so.prods[b];
+            keys += so.keys[b];
+            bound += so.bound[b];
+        }
+        if (2 * bigrows < rows || 2 * wide < rows || keys == 0 || !scatter_fits(c)) return false;
+        // distinct keys of a whole row, from those among the products looked
+        // at: n random columns give n (1 - exp(-p / n)) of p products
+        const double p = (double)prods / bigrows, k = (double)keys / bigrows, u = (double)bound / bigrows;
+        double lo = k, hi = (double)A.N;
+        for (int it = 0; it < 40; it++) {
+            const double n = 0.5 * (lo + hi);
+            if (n * (1.0 - std::exp(-p / n)) < k) lo = n;
+            else hi = n;
+        }
+        return u <= kScatterMerge * hi * (1.0 - std::exp(-u / hi));
+    }
+    bool scatter_fits(Context *c) const
+    {
+        return P.N <= scatter_cap(c->max_lds) && R.M * (int64_t)scatter_slots() * 12 <= ((int64_t)4 << 30);
+    }
+    void use_scatter()
+    {
+        for (int b = big_from; b < thr.nb; b++) cfg[b] = FusedCfg{256, 64, scatter_slots(), 0, 0, true};
+        lscatter = true;
     }
 
     static void take_multipliers(FusedCfg &f, const SampleOut &so)
@@ -1587,7 +1652,11 @@ struct FusedPlan {
         // the binning clears the control block, and its scatter kernel sends
         // the populations to the host while the likely bin already runs
         SP3MM_HIP(hipGetLastError());
-        const bool sampling = may_sample && pred >= 0;
+        // (rows beyond the bins are sampled only to choose k_scatter_direct,
+        // which cannot pay when they have many more products than A has columns)
+        const bool sampling =
+            may_sample && (pred >= 0 || (scatter_fits(c) && (double)R.nnz * ((double)A.nnz / (double)A.M) <=
+                                                                kScatterMerge * (double)R.M * (double)A.N));
         const unsigned long long sseq = sampling ? queue_sample(c, nullptr, nullptr, pred) : 0;
         const unsigned long long seq = c->poll_host ? ++c->poll_seq : 0;
         launch_binning(c, s, seq);
@@ -1605,11 +1674,12 @@ struct FusedPlan {
         if (sampling) {
             SampleOut so;
             if (read_sample(c, sseq, so)) return -1;
-            sampled = apply_sample(c, so);
+            if (wants_scatter(c, so)) use_scatter();
+            else if (pred >= 0) sampled = apply_sample(c, so);
         }
         // the likely bin's slots; without them it runs with the other bins
         // after the read-back (its rows are listed like any bin's)
-        own = can_sample && keep ? -1 : pred;
+        own = (can_sample && keep) || (pred >= 0 && cfg[pred].scatter) ? -1 : pred;
         if (own >= 0) {
             const size_t cap = (size_t)M * cfg[pred].H2;
             pcol = Buf(cap * 4);
@@ -1660,14 +1730,20 @@ struct FusedPlan {
             return -1;
         }
         // long rows in one pass when their slots stay within 1 GiB
-        lcap = window_cap(c->max_lds - 1024);
+        lcap = lscatter ? scatter_slots() : window_cap(c->max_lds - 1024);
         lslots = false;
-        if (nlong > 0 && !ext_out && (size_t)nlong * lcap * 12 <= ((size_t)1 << 30)) {
+        if (nlong > 0 && !ext_out && (lscatter || (size_t)nlong * lcap * 12 <= ((size_t)1 << 30))) {
             lslotn = Buf((size_t)nlong * 4);
             lcol = Buf((size_t)nlong * lcap * 4);
             lval = Buf((size_t)nlong * lcap * 8);
             lslots = lslotn.p && lcol.p && lval.p;
+            if (lscatter && !lslots) {
+                set_error("scratch allocation (%d long rows) failed", nlong);
+                return -1;
+            }
         }
+        bool scattered = lscatter && nlong > 0;
+        for (int i = 0; i < thr.nb; i++) scattered = scattered || (cnt[i] > 0 && cfg[i].scatter);
         if (en0 < 0) en0 = mk(tm);
         for (int i = 0; i < thr.nb; i++)
             if (cnt[i] && i != own) launch_main(c, s, i);
@@ -1680,7 +1756,7 @@ struct FusedPlan {
         // checks the capacity; if a row was retried, a retried row outgrew the
         // output, or a row spilled to the global dense kernel, the exact path
         // below redoes the tail.
-        const bool speculate = nlong == 0 && !mixed && stot > 0 && stot < INT32_MAX;
+        const bool speculate = nlong == 0 && !scattered && !mixed && stot > 0 && stot < INT32_MAX;
         defer_retry = speculate;
         launch_long(c, s, false);
         if (ext_out) {
@@ -1739,6 +1815,7 @@ struct FusedPlan {
         if (read_ctl(c, d(), h)) return -1;
         nretry = h.nretry;
         nspill = h.nspill;
+        nwide = h.nwide;
         built = true;
         if (nspill > 0 && !h.err) {
             if (sws.alloc(dense_blocks(c, nspill), A.N, P.N, true, s)) return -1;
@@ -1885,7 +1962,9 @@ static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3m
         st->main_kernel_launches = launches;
         st->guarded_rows = nf;
         st->guarded_entries = plan.nretry + plan.nlong;  // rows off the hash-table path
-        st->spilled_rows = plan.nspill;
+        for (int i = 0; i < plan.thr.nb; i++)
+            if (plan.cfg[i].scatter) st->guarded_entries += plan.cnt[i];
+        st->spilled_rows = plan.nspill + plan.nwide;
     }
     return 0;
 }

@@ -120,6 +120,14 @@ void launch_window_direct(bool num, int blocks, size_t lds, const SpOperand &R, 
                           double *rowsum, int64_t out_cap, int *err, hipStream_t st, bool f32in,
                           int32_t *slotn = nullptr, int32_t *scol = nullptr, double *sval = nullptr,
                           int cap_rows = 0x7fffffff);
+// rows of thousands of unstructured products whose output columns fit in LDS
+// (see k_scatter_direct); slots of `cap` >= P.N entries (a multiple of 32);
+// *nwide counts the rows whose R*A columns span more than wcap
+int scatter_cap(size_t lds);
+void launch_scatter_direct(int num_cu, const SpOperand &R, const SpOperand &A, const SpOperand &P,
+                           const int32_t *rows, const int *count, int rows_host, int cap, int32_t *rownnz,
+                           int32_t *slotn, int32_t *scol, double *sval, int wcap, int *nwide, int *err,
+                           hipStream_t st, bool f32in);
 void launch_dense_direct(bool num, int blocks, const SpOperand &R, const SpOperand &A, const SpOperand &P,
                          const int32_t *rows, const int *count, const DenseWs &ws, int slog1, int slog2,
                          int32_t *n1out, int32_t *rownnz, const int64_t *crp, int32_t *ccol, double *cval,
@@ -159,18 +167,24 @@ constexpr int kSampleSplit = 8;    // workgroups per sampled row (a share of the
 constexpr int kSampleTab = 64;
 constexpr int kSampleClasses = 5;  // tables of 64 .. 1024 slots are scored
 constexpr int kSampleCand = 256;
+// wide: sampled rows of the bin whose columns spread over more than a quarter
+// of A's rows; prods / keys: stage-1 products looked at and distinct keys
+// among them (until a row's dedup table was full); bound: the rows' bounds.
 struct SampleOut {
     int rows[kMaxBins + 1], n1[kMaxBins + 1], n2[kMaxBins + 1];
+    int wide[kMaxBins + 1], prods[kMaxBins + 1], keys[kMaxBins + 1], bound[kMaxBins + 1];
     int cls[2];
     unsigned mul[2];
 };
 // device scratch of the sampling: a sampled row's bin and key counts, and its
 // score of every candidate
 struct SampleBoard {
-    int bin[kSampleRows], n[2][kSampleRows];
+    int bin[kSampleRows], n[2][kSampleRows], wide[kSampleRows], prods[kSampleRows], keys[kSampleRows], bound[kSampleRows];
     alignas(16) unsigned short score[kSampleRows][2][kSampleCand];
 };
-// rows / count (device): sample a list of rows instead of all of R's
+// rows / count (device): sample a list of rows instead of all of R's.  pred < 0
+// without a list: a row's keys are not counted beyond some thousand products
+// (n1 and n2 are INT32_MAX then; prods / keys still tell how far they merge)
 void launch_sample_rows(const SpOperand &R, const SpOperand &A, const SpOperand &P, const int32_t *rows,
                         const int *count, const BinThresholds &thr, int pred,
                         SampleBoard *board, SampleOut *host, unsigned long long *flag, unsigned long long seq,

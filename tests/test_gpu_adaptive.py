@@ -94,3 +94,37 @@ def test_both_sides_of_the_size_rule(n, path):
     want = O.sp3mm_merged(R, A, P)
     assert np.array_equal(got.irp, want.irp) and np.array_equal(got.ja, want.ja)
     assert O.rel_errors(got, want, O.abs_product(R, A, P)).max() < 1e-12
+
+
+def _random(rng, m, n, lens):
+    """m x n with the given row lengths, columns uniform, values in [-1, 1)."""
+    irp = np.concatenate([[0], np.cumsum(lens)])
+    cols = np.concatenate([np.sort(rng.choice(n, int(k), replace=False)) for k in lens])
+    return CSR(m, n, irp, cols, rng.uniform(-1.0, 1.0, cols.size))
+
+
+@pytest.mark.parametrize("ncol,f32", [(30, False), (64, False), (1000, False), (1000, True), (7521, False),
+                                      (17696, False), (17697, False)])
+def test_unmerged_forwarding(ncol, f32):
+    """Unstructured rows of thousands of products (k_scatter_direct): R rows
+    around the 512 entries staged at once, empty and 2,000-entry rows of A and
+    P, output widths up to the widest the LDS accumulators take and past it."""
+    L.set_tuning(None)
+    rng = np.random.default_rng(ncol)
+    k, j, m = 3000, 21000, 260
+    lr = rng.integers(400, 700, m)
+    lr[:4] = 511, 512, 513, 1024
+    la = rng.integers(0, 50, k)
+    la[::500] = 2000
+    lp = np.minimum(rng.integers(0, 24, j), ncol)
+    lp[::3000] = min(2000, ncol)
+    R, A, P = _random(rng, m, k, lr), _random(rng, k, j, la), _random(rng, j, ncol, lp)
+    if f32:
+        R, A, P = (x.with_vals(x.vals.astype(np.float32).astype(np.float64)) for x in (R, A, P))
+        got, st, _ = L.rap_mixed_host(R, A, P, precision=L.MIXED64)
+    else:
+        got, st = L.rap_host(R, A, P)
+    assert st["guarded_entries"] == m  # no row on the hash tables
+    want = O.sp3mm_pair(R, A, P)
+    assert np.array_equal(got.irp, want.irp) and np.array_equal(got.ja, want.ja)
+    assert np.all(np.abs(got.vals - want.vals) <= O.error_bound(R, A, P, want))
