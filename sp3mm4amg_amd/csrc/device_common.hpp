@@ -23,6 +23,7 @@ enum : int {
     kErrOverflow = 2,     // an output row did not fit the space reserved for it
     kErrBadInput = 4,     // input validation failed
     kErrSpin = 8,         // a bounded wait gave up
+    kErrLongRow = 16,     // a row is longer than the kernel takes (the caller has another path)
 };
 
 __device__ __forceinline__ int lane() { return (int)__lane_id(); }

@@ -405,7 +405,8 @@ struct Ctl {
     int nwide;   // rows of k_scatter_direct whose windows would
     unsigned long long totals[3];  // bound sum, bound maximum, rows of unstructured spread
     int64_t nnz;
-    int64_t pad2;
+    int longest;  // longest row seen (prolongator)
+    int pad2;
 };
 
 static int max_blocks(const Context *c) { return c->num_cu * 16; }
@@ -2184,6 +2185,78 @@ struct SaPlan {
     }
 };
 
+// P = (I - omega D^-1 A) P0 from A's rows and the aggregate ids (k_sa_rows).
+// build() finds the row lengths and fills P, allocated for the most entries
+// it can have (A's and a diagonal per row), and with `replayable` also the
+// longest row (atomics: 75 us on 10^5 rows); record() refills its columns and
+// values for new values of A (same pattern), without host synchronisation.
+// build() returns 1, nothing allocated, when a row of A is longer than the
+// kernel takes (the caller forms S and S P0 instead).
+struct SaRowsPlan {
+    sp3mm_dmat A{}, P{};
+    double omega = 0;
+    int mode = 0;
+    int longest = INT32_MAX;  // longest row of A, once counted
+    Buf ctl, agg;
+    Ctl *d() const { return ctl.as<Ctl>(); }
+
+    int build(Context *c, const sp3mm_dmat &a, const int64_t *host_agg, int64_t nagg, double om, int md,
+              bool replayable)
+    {
+        A = a;
+        omega = om;
+        mode = md;
+        const int64_t M = A.M;
+        if (A.nnz + M >= INT32_MAX) return 1;
+        hipStream_t s = c->stream;
+        ctl = Buf(sizeof(Ctl));
+        agg = Buf((size_t)(M ? M : 1) * 4);
+        Buf wide((size_t)(M ? M : 1) * 8), len((size_t)(M + 1) * 4), tiles((size_t)scan_tiles(M) * 8);
+        if (!ctl.p || !agg.p || !wide.p || !len.p || !tiles.p) {
+            set_error("prolongator: scratch allocation failed");
+            return -1;
+        }
+        launch_fill_i32(reinterpret_cast<int32_t *>(d()), (int64_t)(sizeof(Ctl) / 4), 0, s);
+        if (M) SP3MM_HIP(hipMemcpyAsync(wide.p, host_agg, (size_t)M * 8, hipMemcpyHostToDevice, s));
+        launch_agg_narrow(wide.as<int64_t>(), M, nagg, agg.as<int32_t>(), &d()->err, s);
+        if (dmat_alloc(P, M, nagg, A.nnz + M, SP3MM_F64)) {
+            dmat_release(P);
+            return -1;
+        }
+        launch_sa_rows(false, A.rp, A.col, static_cast<const double *>(A.val), agg.as<int32_t>(), M, A.nnz, omega,
+                       mode, nullptr, len.as<int32_t>(), nullptr, nullptr, replayable ? &d()->longest : nullptr, INT32_MAX,
+                       &d()->err, s);
+        launch_scan(len.as<int32_t>(), M, P.rp, P.rp32, tiles.as<long long>(), &d()->nnz, s);
+        fill(s);
+        Ctl h;
+        if (read_ctl(c, d(), h)) {
+            dmat_release(P);
+            return -1;
+        }
+        if (h.err) dmat_release(P);
+        if (h.err == kErrLongRow) return 1;
+        if (h.err) {
+            set_error("prolongator: %s (zero diagonal, or an aggregate out of range)", err_text(h.err & ~kErrLongRow));
+            return -1;
+        }
+        P.nnz = h.nnz;
+        if (replayable) longest = h.longest;
+        return 0;
+    }
+
+    void fill(hipStream_t s)
+    {
+        launch_sa_rows(true, A.rp, A.col, static_cast<const double *>(A.val), agg.as<int32_t>(), A.M, A.nnz, omega,
+                       mode, P.rp, nullptr, P.col, static_cast<double *>(P.val), nullptr, longest, &d()->err, s);
+    }
+
+    void record(Context *, hipStream_t s)
+    {
+        launch_fill_i32(&d()->err, 1, 0, s);
+        fill(s);
+    }
+};
+
 int sa_prolongator(const sp3mm_dmat &A, const int64_t *agg, int64_t nagg, double omega, int mode, sp3mm_dmat &P)
 {
     Context *c = ctx();
@@ -2200,6 +2273,12 @@ int sa_prolongator(const sp3mm_dmat &A, const int64_t *agg, int64_t nagg, double
     if (nagg <= 0 || nagg >= INT32_MAX || (mode != 0 && mode != 1)) {
         set_error("prolongator: bad aggregate count or diagonal mode");
         return -1;
+    }
+    {
+        SaRowsPlan rows;
+        const int rc = rows.build(c, A, agg, nagg, omega, mode, false);
+        if (rc == 0) P = rows.P;
+        if (rc <= 0) return rc;
     }
     hipStream_t s = c->stream;
     const int64_t M = A.M;
@@ -3164,21 +3243,29 @@ void batch_free(void *h)
 // that the whole chain is captured as one HIP graph and replayed when A_0's
 // values change (its pattern must not: a fingerprint of it is checked first).
 struct HierLevel {
-    SaPlan sa;
+    SaRowsPlan rows;    // P from A's rows, or
+    bool by_rows = false;
+    SaPlan sa;          // S, and
     sp3mm_dmat I{}, P0{};
-    FusedPlan pplan;    // P = I * S * P0
+    FusedPlan pplan;    // P = I * S * P0 (a row of A_l is too long for `rows`)
     TransposePlan tr;   // R = P^T
     FusedPlan rap;      // A_{l+1} = R * A_l * P
+    const sp3mm_dmat &P() const { return by_rows ? rows.P : pplan.C; }
 
     void record(Context *c, hipStream_t s)
     {
-        sa.record(c, s);
-        pplan.record(c, s);
+        if (by_rows) {
+            rows.record(c, s);
+        } else {
+            sa.record(c, s);
+            pplan.record(c, s);
+        }
         tr.record(c, s);
         rap.record(c, s);
     }
     void release_all()
     {
+        dmat_release(rows.P);
         dmat_release(sa.S);
         dmat_release(I);
         dmat_release(P0);
@@ -3276,36 +3363,48 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
         }
         h->lv.emplace_back(new HierLevel());
         HierLevel &L = *h->lv.back();
-        std::vector<int64_t> iota((size_t)M);
-        for (int64_t i = 0; i < M; i++) iota[(size_t)i] = i;
-        Buf dagg((size_t)(M ? M : 1) * 8), diota((size_t)(M ? M : 1) * 8);
-        if (!dagg.p || !diota.p) {
-            set_error("hierarchy: allocation failed");
-            hier_release(h);
-            return nullptr;
-        }
-        if (hip_failed(hipMemcpyAsync(dagg.p, aggs[l], (size_t)M * 8, hipMemcpyHostToDevice, c->stream)) ||
-            hip_failed(hipMemcpyAsync(diota.p, iota.data(), (size_t)M * 8, hipMemcpyHostToDevice, c->stream)) ||
-            L.sa.build(c, cur, omega, mode) || one_per_row(c, dagg.as<int64_t>(), M, nagg, L.P0, ctl) ||
-            one_per_row(c, diota.as<int64_t>(), M, M, L.I, ctl)) {
-            hier_release(h);
-            return nullptr;
-        }
         Timer t2(c->stream, false);
-        L.pplan.R = L.I;
-        L.pplan.A = L.sa.S;
-        L.pplan.P = L.P0;
-        // with the identity on the left, a row's bound is its exact distinct
-        // count: a table of twice the bound keeps probe sequences short
-        L.pplan.tu = c->tune;
-        L.pplan.tu.h1_shift = -1;
-        if (L.pplan.build(c, t2) || L.tr.build(c, L.pplan.C, true)) {
+        const int rc = L.rows.build(c, cur, aggs[l], nagg, omega, mode, true);
+        L.by_rows = rc == 0;
+        if (rc < 0) {
+            hier_release(h);
+            return nullptr;
+        }
+        if (!L.by_rows) {
+            std::vector<int64_t> iota((size_t)M);
+            for (int64_t i = 0; i < M; i++) iota[(size_t)i] = i;
+            Buf dagg((size_t)(M ? M : 1) * 8), diota((size_t)(M ? M : 1) * 8);
+            if (!dagg.p || !diota.p) {
+                set_error("hierarchy: allocation failed");
+                hier_release(h);
+                return nullptr;
+            }
+            if (hip_failed(hipMemcpyAsync(dagg.p, aggs[l], (size_t)M * 8, hipMemcpyHostToDevice, c->stream)) ||
+                hip_failed(hipMemcpyAsync(diota.p, iota.data(), (size_t)M * 8, hipMemcpyHostToDevice, c->stream)) ||
+                L.sa.build(c, cur, omega, mode) || one_per_row(c, dagg.as<int64_t>(), M, nagg, L.P0, ctl) ||
+                one_per_row(c, diota.as<int64_t>(), M, M, L.I, ctl)) {
+                hier_release(h);
+                return nullptr;
+            }
+            L.pplan.R = L.I;
+            L.pplan.A = L.sa.S;
+            L.pplan.P = L.P0;
+            // with the identity on the left, a row's bound is its exact distinct
+            // count: a table of twice the bound keeps probe sequences short
+            L.pplan.tu = c->tune;
+            L.pplan.tu.h1_shift = -1;
+            if (L.pplan.build(c, t2)) {
+                hier_release(h);
+                return nullptr;
+            }
+        }
+        if (L.tr.build(c, L.P(), true)) {
             hier_release(h);
             return nullptr;
         }
         L.rap.R = L.tr.T;
         L.rap.A = cur;
-        L.rap.P = L.pplan.C;
+        L.rap.P = L.P();
         L.rap.tu = c->tune;
         L.rap.adapt = c->adapt;
         L.rap.keep = true;
@@ -3318,8 +3417,12 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
     // the error words every replay must leave clear
     std::vector<const int *> words;
     for (auto &l : h->lv) {
-        words.push_back(&l->sa.d()->err);
-        words.push_back(&l->pplan.d()->err);
+        if (l->by_rows) {
+            words.push_back(&l->rows.d()->err);
+        } else {
+            words.push_back(&l->sa.d()->err);
+            words.push_back(&l->pplan.d()->err);
+        }
         words.push_back(&l->rap.d()->err);
     }
     h->nerr = (int)words.size();
@@ -3406,7 +3509,7 @@ int hier_level(void *hp, int l, sp3mm_dmat &R, sp3mm_dmat &P, sp3mm_dmat &Ac)
     }
     HierLevel &L = *h->lv[(size_t)l];
     R = L.tr.T;
-    P = L.pplan.C;
+    P = L.P();
     Ac = L.rap.C;
     R.owned = P.owned = Ac.owned = 0;
     return 0;

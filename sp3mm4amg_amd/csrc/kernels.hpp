@@ -271,6 +271,15 @@ void launch_sa_fill(const int64_t *rp, const int32_t *col, const double *val, in
                     int mode, const int64_t *srp, int32_t *scol, double *sval, int *err, hipStream_t st);
 void launch_p0_fill(const int64_t *agg, int64_t M, int64_t nagg, int64_t *rp, int32_t *rp32, int32_t *col,
                     double *val, int *err, hipStream_t st);
+// P = (I - omega D^-1 A) P0 row by row (see k_sa_rows): aggregate ids narrowed
+// and checked, row lengths, then columns and values at the offsets prp.  *err
+// receives kErrLongRow if a row of A is longer than the kernel takes, *maxlen
+// (fill = false) the longest row of A that was not taken in registers;
+// longest: that value for a pattern that was counted, INT32_MAX otherwise.
+void launch_agg_narrow(const int64_t *agg, int64_t M, int64_t nagg, int32_t *out, int *err, hipStream_t st);
+void launch_sa_rows(bool fill, const int64_t *rp, const int32_t *col, const double *val, const int32_t *agg, int64_t M,
+                    int64_t nnz, double omega, int mode, const int64_t *prp, int32_t *len, int32_t *pcol,
+                    double *pval, int *maxlen, int longest, int *err, hipStream_t st);
 void launch_spmv(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz, const double *x,
                  const double *z, double *y, double alpha, double beta, hipStream_t st);
 // all sweeps in one workgroup when the system fits in max_lds bytes of LDS

@@ -3,6 +3,7 @@
 // prolongator P = (I - omega D^-1 A) P0 (P0 = the 0/1 aggregation matrix).
 // The reference receives P and R from its caller; these kernels let a whole
 // hierarchy be built level after level without leaving HBM.
+#include <algorithm>
 #include <cstdlib>
 
 #include "device_common.hpp"
@@ -216,6 +217,177 @@ __global__ void k_p0_fill(const int64_t *__restrict__ agg, int64_t M, int64_t na
     }
 }
 
+__global__ void k_agg_narrow(const int64_t *__restrict__ agg, int64_t M, int64_t nagg, int32_t *__restrict__ out,
+                             int *__restrict__ err)
+{
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < M; r += stride) {
+        const int64_t a = agg[r];
+        const bool ok = a >= 0 && a < nagg;
+        if (!ok) atomicOr(err, kErrBadInput);
+        out[r] = ok ? (int32_t)a : 0;
+    }
+}
+
+// Row r of P = (I - omega D^-1 A) P0 straight from row r of A: entry (r, k)
+// contributes -omega a_rk / d_r (+ 1 on the diagonal, which counts as stored)
+// to column agg[k], equal columns added in increasing k.  FILL = false: row
+// lengths only.
+// L = 8: rows of at most 8 entries (diagonal included) sit in 8 lanes, one
+// entry each; every lane compares its aggregate with the others' by shuffles,
+// so a row costs 16 shuffles and no LDS, and 8 rows share a wavefront.
+// Longer rows (all of them with L = 64) take the whole wavefront and an LDS
+// hash table of up to CAP slots, keyed by the aggregate; a row of CAP entries
+// or more raises kErrLongRow.  (Comparing all pairs of a row staged in LDS
+// took 2.2 ms on the coarse levels of a 96^3 hierarchy, the tables 0.06.)
+// It replaces S = I - omega D^-1 A in HBM and the SpGEMM S P0 (count, scan,
+// fill, P0, binning, hash kernel, scan, gather): HBM-bound, 12 bytes per entry
+// of A and of P per pass, the gathers of agg stay in L2.  96^3 7-point
+// operator: 0.70 -> 0.057 ms per recomputation.
+template <int L, int CAP, bool FILL>
+__global__ void __launch_bounds__(256) k_sa_rows(const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                  const double *__restrict__ val, const int32_t *__restrict__ agg,
+                                                  int64_t M, double omega, int mode, const int64_t *__restrict__ prp,
+                                                  int32_t *__restrict__ len, int32_t *__restrict__ pcol,
+                                                  double *__restrict__ pval, int *__restrict__ maxlen,
+                                                  int *__restrict__ err)
+{
+    __shared__ double sv[4][FILL ? CAP : 1];
+    __shared__ int sk[4][CAP];
+    static_assert(L == 8 || L == kWave, "register rows of 8 lanes, or wavefronts");
+    const int wv = threadIdx.x / kWave, l = lane(), sub = l & (L - 1), lead = l & ~(L - 1);
+    constexpr int RPW = kWave / L;  // rows per wavefront
+    const uint64_t part = L == kWave ? ~0ull : ((1ull << L) - 1) << lead;
+    const int64_t stride = (int64_t)gridDim.x * 4 * RPW;
+    int longest = 0;
+    for (int64_t r0 = ((int64_t)blockIdx.x * 4 + wv) * RPW; r0 < M; r0 += stride) {
+        const int64_t r = r0 + l / L;
+        const int64_t b = r < M ? rp[r] : 0;
+        const int64_t n64 = r < M ? rp[r + 1] - b : 0;
+        const bool fits = L < kWave && n64 <= L;
+        const int n = fits ? (int)n64 : 0;
+        int c = -1;
+        double v = 0.0;
+        if (sub < n) {
+            c = col[b + sub];
+            if (FILL) v = val[b + sub];
+        }
+        const bool isd = sub < n && c == r;
+        const bool has = (ballot(isd) & part) != 0;
+        const int m = r < M && fits ? n + (has ? 0 : 1) : 0;  // entries with the diagonal
+        const bool is_long = r < M && (!fits || m > L);
+        if (sub == n && m == n + 1 && m <= L) c = (int)r;  // the missing diagonal
+        const bool act = sub < m && m <= L;
+        const int key = act ? agg[c] : INT32_MAX;
+        double s = 0.0;
+        bool bad = false;
+        if (FILL) {
+            double d = isd ? v : 0.0;
+            for (int o = L / 2; o > 0; o >>= 1) d += __shfl_xor(d, o, L);
+            if (mode == 1) d = fabs(d) + 1.0;
+            bad = act && d == 0.0;
+            if (bad) atomicOr(err, kErrBadInput);
+            else if (act) s = -(omega / d) * v + (c == r ? 1.0 : 0.0);
+        }
+        bool first = act;
+        double sum = 0.0;
+#pragma unroll 8
+        for (int i = 0; i < L; i++) {
+            const int ki = __shfl(key, i, L);
+            if (FILL) {
+                const double si = __shfl(s, i, L);
+                if (ki == key) sum += si;
+            }
+            if (ki == key && i < sub) first = false;
+        }
+        const uint64_t fm = ballot(first) & part;
+        if (!FILL) {
+            if (sub == 0 && r < M && !is_long) len[r] = __popcll(fm);
+        } else {
+            const uint64_t fl = fm >> lead;
+            int rank = 0;
+#pragma unroll 8
+            for (int i = 0; i < L; i++) {
+                const int ki = __shfl(key, i, L);
+                rank += ((fl >> i) & 1) && ki < key;
+            }
+            if (first && !bad) {
+                const int64_t o = prp[r] + rank;
+                pcol[o] = key;
+                pval[o] = sum;
+            }
+        }
+        // rows beyond L lanes, one after the other
+        for (uint64_t lm = ballot(is_long && sub == 0); lm; lm &= lm - 1) {
+            const int64_t q = r0 + (__ffsll((unsigned long long)lm) - 1) / L;
+            const int64_t qb = rp[q];
+            const int64_t qn = rp[q + 1] - qb;
+            if (!FILL) longest = max(longest, (int)min(qn, (int64_t)INT32_MAX));
+            if (qn + 1 > CAP) {
+                if (l == 0) atomicOr(err, kErrLongRow);
+                if (!FILL && l == 0) len[q] = 0;
+                continue;
+            }
+            // a table of at least the row's entries, 4/3 of them up to CAP
+            int H = kWave, lg = 6;
+            while (H < CAP && 3 * H < 4 * ((int)qn + 1)) {
+                H *= 2;
+                lg++;
+            }
+            int *k = sk[wv];
+            double *s2 = sv[wv];
+            for (int i = l; i < H; i += kWave) {
+                k[i] = kEmpty;
+                if (FILL) s2[i] = 0.0;
+            }
+            double w = 0.0;
+            bool hd = false;  // the diagonal is stored
+            for (int64_t e0 = qb; e0 < qb + qn; e0 += kWave) {
+                const bool at = e0 + l < qb + qn && col[min(e0 + l, qb + qn - 1)] == q;
+                const uint64_t am = ballot(at);
+                if (am) {
+                    hd = true;
+                    if (FILL) w = val[e0 + __ffsll((unsigned long long)am) - 1];
+                    break;
+                }
+            }
+            if (FILL) {
+                if (mode == 1) w = fabs(w) + 1.0;
+                if (w == 0.0) {
+                    if (l == 0) atomicOr(err, kErrBadInput);
+                    continue;
+                }
+                w = omega / w;
+            }
+            wave_sync();
+            int nd = 0;
+            for (int e = l; e < (int)qn + (hd ? 0 : 1); e += kWave) {
+                const int ce = e < (int)qn ? col[qb + e] : (int)q;
+                int fresh = 0;
+                const int at = hash_insert(k, (unsigned)H - 1, 32 - lg, agg[ce], &fresh);
+                nd += fresh;
+                if (FILL) atomicAdd(s2 + at, -w * (e < (int)qn ? val[qb + e] : 0.0) + (ce == q ? 1.0 : 0.0));
+            }
+            wave_sync();
+            if (!FILL) {
+                for (int o = 32; o > 0; o >>= 1) nd += __shfl_xor(nd, o);
+                if (l == 0) len[q] = nd;
+            } else {
+                const int n2 = compact_table<kWave, double>(k, s2, H, nullptr);
+                const int64_t o = prp[q];
+                for (int j = l; j < n2; j += kWave) {
+                    const int rank = key_rank(k, n2, k[j]);
+                    pcol[o + rank] = k[j];
+                    pval[o + rank] = s2[j];
+                }
+            }
+            wave_sync();
+        }
+    }
+    if (!FILL && maxlen && l == 0 && longest > __hip_atomic_load(maxlen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(maxlen, longest);
+}
+
 static unsigned grid1(int64_t n, int threads = 256)
 {
     int64_t b = (n + threads - 1) / threads;
@@ -233,7 +405,11 @@ void launch_transpose_scatter(const int64_t *rp, const int32_t *col, const void 
                               int32_t *tsrc, hipStream_t st)
 {
     if (M == 0) return;
-    const int L = lanes_for(M, nnz);
+    // every entry waits for a returning atomic: rows of four entries take four
+    // lanes (1.5e6 entries: 72 us with one lane per row, 28 with four); longer
+    // rows stay at four entries per lane (rows of 9 and 70: 19 and 37 us, a
+    // lane per entry 62 and 39: more of the counters' rows are hit at once)
+    const int L = std::max(lanes_for(M, nnz), nnz >= 3 * M ? 4 : 1);
     const unsigned g = grid1(M, 256 / L);
     if (f32) {
         const float *v = static_cast<const float *>(val);
@@ -306,6 +482,39 @@ void launch_p0_fill(const int64_t *agg, int64_t M, int64_t nagg, int64_t *rp, in
                     double *val, int *err, hipStream_t st)
 {
     hipLaunchKernelGGL(k_p0_fill, dim3(grid1(M + 1)), dim3(256), 0, st, agg, M, nagg, rp, rp32, col, val, err);
+}
+
+void launch_agg_narrow(const int64_t *agg, int64_t M, int64_t nagg, int32_t *out, int *err, hipStream_t st)
+{
+    if (M > 0) hipLaunchKernelGGL(k_agg_narrow, dim3(grid1(M)), dim3(256), 0, st, agg, M, nagg, out, err);
+}
+
+// lanes by the mean row (a 7-point row and a missing diagonal fit 8 lanes;
+// operators of longer rows run a wavefront per row); tables for the longest
+// row when it is known (four of 1024 slots leave 12 wavefronts per CU: second
+// level of a 96^3 hierarchy, 110,592 rows of 33, 125 us against 59)
+void launch_sa_rows(bool fill, const int64_t *rp, const int32_t *col, const double *val, const int32_t *agg, int64_t M,
+                    int64_t nnz, double omega, int mode, const int64_t *prp, int32_t *len, int32_t *pcol,
+                    double *pval, int *maxlen, int longest, int *err, hipStream_t st)
+{
+    if (M == 0) return;
+    const double avg = (double)nnz / (double)M;
+    const int L = avg <= 8 ? 8 : kWave;
+    const unsigned g = grid1(M, 4 * (kWave / L));
+#define SP3MM_SA_ROWS(LL, CC)                                                                                      \
+    do {                                                                                                           \
+        if (fill)                                                                                                  \
+            hipLaunchKernelGGL((k_sa_rows<LL, CC, true>), dim3(g), dim3(256), 0, st, rp, col, val, agg, M, omega,  \
+                               mode, prp, len, pcol, pval, maxlen, err);                                                  \
+        else                                                                                                       \
+            hipLaunchKernelGGL((k_sa_rows<LL, CC, false>), dim3(g), dim3(256), 0, st, rp, col, val, agg, M, omega, \
+                               mode, prp, len, pcol, pval, maxlen, err);                                                  \
+    } while (0)
+    if (L == 8) SP3MM_SA_ROWS(8, 128);
+    else if (longest < 128) SP3MM_SA_ROWS(64, 128);
+    else if (longest < 512) SP3MM_SA_ROWS(64, 512);
+    else SP3MM_SA_ROWS(64, 1024);
+#undef SP3MM_SA_ROWS
 }
 
 }  // namespace sp3mm
