@@ -2880,12 +2880,27 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
             endb_ms = ms1;
         }
     }
-    cur = endb;
-    cur_ms = endb_ms;
-    c->tune = cur;
+    // the choice against the start once more, interleaved: a start that is not
+    // slower stays (the two were timed minutes of products apart)
+    if (!same_tuning(endb, saved)) {
+        double ms_end = 0;
+        if (confirm(saved, endb, ms_default, ms_end)) {
+            c->tune = saved;
+            return -1;
+        }
+        if (ms_end < ms_default) {
+            endb_ms = ms_end;
+        } else {
+            endb = saved;
+            endb_ms = ms_default;
+        }
+    } else {
+        endb_ms = ms_default;
+    }
+    c->tune = endb;
     fixed.was = false;
-    best = cur;
-    ms_best = cur_ms;
+    best = endb;
+    ms_best = endb_ms;
     return 0;
 }
 
