@@ -2352,7 +2352,7 @@ int set_stream(hipStream_t s)
 ConsState *cons_state(Context *c)
 {
     if (!c->cons) {
-        const size_t bytes = sizeof(ConsState) + (size_t)dot_parts() * 8;
+        const size_t bytes = sizeof(ConsState) + (size_t)dot_parts() * 8 + jacobi_grid_bytes();
         if (hipMalloc(&c->cons, bytes) != hipSuccess) {
             (void)hipGetLastError();
             c->cons = nullptr;
@@ -2367,6 +2367,12 @@ ConsState *cons_state(Context *c)
     return static_cast<ConsState *>(c->cons);
 }
 
+// x buffers of launch_jacobi_grid, behind the dot's partial sums
+static void *jacobi_buffers(Context *c)
+{
+    return c->cons ? static_cast<unsigned char *>(c->cons) + sizeof(ConsState) + (size_t)dot_parts() * 8 : nullptr;
+}
+
 int consumer_wait(Context *c, double *dot_out)
 {
     if (!c->cons) {
@@ -2374,14 +2380,25 @@ int consumer_wait(Context *c, double *dot_out)
         return 0;
     }
     ConsState h{};
-    SP3MM_HIP(hipMemcpyAsync(&h, c->cons, sizeof h, hipMemcpyDeviceToHost, c->stream));
-    SP3MM_HIP(hipStreamSynchronize(c->stream));
+    static_assert(sizeof(ConsState) % 4 == 0, "exported as words");
+    if (c->host_small_dev) {
+        // a copy into pageable memory and a blocking wait left the GPU idle
+        // for 37 us between the cycles of a solve
+        launch_export_words(c->cons, c->host_small_dev, (int)(sizeof h / 4), c->stream);
+        SP3MM_HIP(hipGetLastError());
+        SP3MM_HIP(spin_stream(c->stream));
+        memcpy(&h, c->host_small, sizeof h);
+    } else {
+        SP3MM_HIP(hipMemcpyAsync(&h, c->cons, sizeof h, hipMemcpyDeviceToHost, c->stream));
+        SP3MM_HIP(hipStreamSynchronize(c->stream));
+    }
     if (dot_out) *dot_out = h.dot;
     if (h.err) {
         ConsState *d = static_cast<ConsState *>(c->cons);
         SP3MM_HIP(hipMemsetAsync(&d->err, 0, sizeof(int), c->stream));
         SP3MM_HIP(hipStreamSynchronize(c->stream));
-        set_error("jacobi: zero diagonal entry (sweep launched before this call)");
+        if (h.err & kErrSpin) set_error("jacobi: a sweep waited in vain for another workgroup's rows");
+        else set_error("jacobi: zero diagonal entry (sweep launched before this call)");
         return -1;
     }
     return 0;
@@ -2457,14 +2474,27 @@ int jacobi(const sp3mm_dmat &A, const double *b, double *x, double *work, double
 }
 
 void queue_jacobi(const sp3mm_dmat &A, const double *b, double *x, double *work, double omega, int sweeps, int *err,
-                  hipStream_t s)
+                  hipStream_t s, bool from_zero)
 {
     const double *val = static_cast<const double *>(A.val);
-    if (sweeps > 1 && launch_jacobi_small(A.rp, A.col, val, A.M, A.nnz, b, x, omega, sweeps, err,
-                                          ctx()->lds_device, s))
+    const bool small = sweeps > 1 && jacobi_small_fits(A.M, A.nnz, ctx()->lds_device);
+    if (!small && launch_jacobi_grid(A.rp, A.col, val, A.M, A.nnz, b, x, jacobi_buffers(ctx()), omega, sweeps,
+                                     from_zero, err, s))
         return;
+    if (from_zero && (small || sweeps == 0)) launch_axpby(A.M, 0.0, nullptr, 0.0, x, s);
+    if (small) {
+        launch_jacobi_small(A.rp, A.col, val, A.M, A.nnz, b, x, omega, sweeps, err, ctx()->lds_device, s);
+        return;
+    }
     double *cur = x, *nxt = work;
-    for (int k = 0; k < sweeps; k++) {
+    int k = 0;
+    if (from_zero && sweeps > 0) {
+        // the first sweep goes where the last one ends in x
+        if ((sweeps - 1) % 2) std::swap(cur, nxt);
+        launch_jacobi_zero(A.rp, A.col, val, A.M, b, cur, omega, err, s);
+        k = 1;
+    }
+    for (; k < sweeps; k++) {
         launch_jacobi(A.rp, A.col, val, A.M, A.nnz, b, cur, nxt, omega, err, s);
         std::swap(cur, nxt);
     }

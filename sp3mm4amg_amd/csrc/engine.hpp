@@ -79,7 +79,8 @@ struct Context {
 
 // Device state of the level consumers: the last dot result, a sticky error
 // word that Jacobi sweeps set on a zero diagonal entry, then the dot's
-// partial sums.  Allocated on first use.
+// partial sums and the sweeps' x vectors of launch_jacobi_grid.  Allocated on
+// first use.
 struct ConsState {
     double dot;
     int err;
@@ -101,9 +102,10 @@ int hash_scores(Context *c, const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3m
                 const int32_t *rows, int nrows, std::vector<unsigned long long> &h, std::vector<int> *nkeys);
 hipError_t spin_event(hipEvent_t e);
 
-// Queues `sweeps` damped Jacobi sweeps (x in place, work as the other buffer).
+// Queues `sweeps` damped Jacobi sweeps (x in place, work as the other buffer);
+// from_zero: the sweeps start from x = 0, whatever x holds.
 void queue_jacobi(const sp3mm_dmat &A, const double *b, double *x, double *work, double omega, int sweeps, int *err,
-                  hipStream_t s);
+                  hipStream_t s, bool from_zero = false);
 
 Context *ctx();  // initialised on first use (device 0 unless sp3mm_init chose one)
 

@@ -282,8 +282,17 @@ void launch_sa_rows(bool fill, const int64_t *rp, const int32_t *col, const doub
                     double *pval, int *maxlen, int longest, int *err, hipStream_t st);
 void launch_spmv(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz, const double *x,
                  const double *z, double *y, double alpha, double beta, hipStream_t st);
-// all sweeps in one workgroup when the system fits in max_lds bytes of LDS
-// (returns false, launching nothing, otherwise)
+// all sweeps in one launch over several workgroups, or in one workgroup when
+// the system fits in max_lds bytes of LDS (return false, launching nothing,
+// otherwise)
+bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
+                        const double *b, double *x, void *buf, double omega, int sweeps, bool from_zero, int *err,
+                        hipStream_t st);
+size_t jacobi_grid_bytes();  // of `buf`
+bool jacobi_small_fits(int64_t M, int64_t nnz, size_t max_lds);
+// one sweep from x = 0 into xo
+void launch_jacobi_zero(const int64_t *rp, const int32_t *col, const double *val, int64_t M, const double *b,
+                        double *xo, double omega, int *err, hipStream_t st);
 bool launch_jacobi_small(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
                          const double *b, double *x, double omega, int sweeps, int *err, size_t max_lds,
                          hipStream_t st);

@@ -611,6 +611,34 @@ __global__ void __launch_bounds__(256) k_jacobi(const int64_t *__restrict__ rp, 
     }
 }
 
+// The first sweep from x = 0: xo = omega b / a_ii.  Only the diagonal is read
+// (found by bisection in the row's sorted columns), not the row: 4.8 us of
+// clearing x and 34 us of sweep against 23 us on 262,144 rows of 32 entries,
+// 4.5 + 23 against 7 on 32,768 rows of 180.
+__global__ void __launch_bounds__(256) k_jacobi_zero(const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                      const double *__restrict__ val, int64_t M,
+                                                      const double *__restrict__ b, double *__restrict__ xo,
+                                                      double omega, int *__restrict__ err)
+{
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= M) return;
+    const int64_t e1 = rp[r + 1];
+    int64_t lo = rp[r], n = e1 - lo;
+    const double br = b[r];
+    while (n > 0) {  // the first column not below r
+        const int64_t h = n / 2;
+        if (col[lo + h] < r) {
+            lo += h + 1;
+            n -= h + 1;
+        } else {
+            n = h;
+        }
+    }
+    const double d = lo < e1 && col[lo] == r ? val[lo] : 0.0;
+    if (d == 0.0) atomicOr(err, kErrBadInput);
+    else xo[r] = 0.0 + omega * (br - 0.0) / d;
+}
+
 // All `sweeps` sweeps of a small system in one workgroup, with the matrix,
 // b and both x vectors staged in LDS once (a coarsest-level solve is a few
 // kilobytes; a launch per sweep would cost more than the sweep).  Rows are
@@ -669,6 +697,106 @@ __global__ void __launch_bounds__(1024) k_jacobi_small(const int64_t *__restrict
 
 static size_t jacobi_small_lds(int64_t M, int64_t nnz) { return (size_t)nnz * 12 + (size_t)M * 24 + (size_t)(M + 1) * 4; }
 
+// All `sweeps` sweeps of a medium system (M up to kGridRows rows, too large for
+// one workgroup's LDS) in one launch: a launch per sweep costs 6.6 us on a
+// 512-row operator of 300 entries per row, several times the sweep itself.
+// Every L-lane group keeps one row in registers (kGridRegs entries per lane,
+// what is beyond them is read again in every sweep) for all sweeps; a
+// workgroup's rows see the whole x of the sweep in LDS.  Sweep k writes its x
+// to buffer k, which starts filled with a signalling NaN no arithmetic
+// produces (hardware quiets NaN results), and the next sweep polls every entry
+// until it is there: the data is its own flag, so a sweep costs one store
+// reaching one load (agent scope) and no barrier across workgroups.  The last
+// sweep writes x.  At most 256 workgroups of 512 lanes and 34 KB of LDS: all
+// fit the 256 CUs at once, and a poll that does not see its entry within
+// kGridSpins loads gives up with kErrSpin, so every wave ends.  Rows are
+// summed in k_jacobi's order (equal results).  50 sweeps in a V-cycle's graph,
+// 512 rows: 330 -> 163 us; called alone 267 -> 183, 1,000 rows 255 -> 223.
+// Two or four rows per group (fewer workgroups polling): 192 to 525 us.
+constexpr int kGridRows = 2048, kGridThreads = 512, kGridRegs = 8, kGridSweeps = 64;
+constexpr unsigned long long kGridEmpty = 0x7FF7A5A57FF7A5A5ull;
+constexpr int kGridSpins = 1 << 21;
+
+template <int L>
+__global__ void __launch_bounds__(kGridThreads) k_jacobi_grid(const int64_t *__restrict__ rp,
+                                                              const int32_t *__restrict__ col,
+                                                              const double *__restrict__ val, int M,
+                                                              const double *__restrict__ b, double *x,
+                                                              unsigned long long *buf, double omega, int sweeps,
+                                                              bool from_zero, int *__restrict__ err)
+{
+    __shared__ double xs[2][kGridRows];
+    __shared__ int dead;
+    const int t = threadIdx.x, sub = t & (L - 1);
+    const int r = blockIdx.x * (kGridThreads / L) + t / L;
+    const bool act = r < M;
+    const int64_t e0 = act ? rp[r] : 0;
+    const int64_t e1 = act ? rp[r + 1] : 0;
+    // this lane's first entries of the row, its right-hand side and diagonal
+    int c[kGridRegs];
+    double v[kGridRegs];
+    double d = 0.0;
+#pragma unroll
+    for (int u = 0; u < kGridRegs; u++) {
+        const int64_t e = e0 + sub + (int64_t)u * L;
+        c[u] = e < e1 ? col[e] : -1;
+        v[u] = e < e1 ? val[e] : 0.0;
+        if (c[u] == r) d = v[u];
+    }
+    for (int64_t e = e0 + sub + (int64_t)kGridRegs * L; e < e1; e += L)
+        if (col[e] == r) d = val[e];
+    for (int o = L / 2; o > 0; o >>= 1) d += __shfl_xor(d, o);
+    const double br = act ? b[r] : 0.0;
+    if (act && sub == 0 && d == 0.0) atomicOr(err, kErrBadInput);
+    if (t == 0) dead = 0;
+    for (int i = t; i < M; i += kGridThreads) xs[0][i] = from_zero ? 0.0 : x[i];
+    __syncthreads();
+    for (int k = 0; k < sweeps; k++) {
+        const double *xi = xs[k & 1];
+        double s = 0.0;
+#pragma unroll
+        for (int u = 0; u < kGridRegs; u++)
+            if (c[u] >= 0) s += v[u] * xi[c[u]];
+        for (int64_t e = e0 + sub + (int64_t)kGridRegs * L; e < e1; e += L) s += val[e] * xi[col[e]];
+        for (int o = L / 2; o > 0; o >>= 1) s += __shfl_xor(s, o);
+        const bool last = k + 1 == sweeps;
+        if (act && sub == 0) {
+            const double xn = d == 0.0 ? xi[r] : xi[r] + omega * (br - s) / d;
+            if (last) x[r] = xn;
+            else
+                __hip_atomic_store(buf + (int64_t)k * M + r, (unsigned long long)__double_as_longlong(xn),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (last) break;
+        // the other buffer of x: nobody reads it any more (sweep k - 1 ended
+        // at the barrier below)
+        double *xo = xs[(k + 1) & 1];
+        for (int i = t; i < M; i += kGridThreads) {
+            unsigned long long w = kGridEmpty;
+            for (int n = 0; n < kGridSpins; n++) {
+                w = __hip_atomic_load(buf + (int64_t)k * M + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (w != kGridEmpty) break;
+                __builtin_amdgcn_s_sleep(1);
+            }
+            if (w == kGridEmpty) dead = 1;
+            xo[i] = __longlong_as_double((long long)w);
+        }
+        __syncthreads();
+        if (dead) {  // uniform: written before the barrier
+            if (t == 0) atomicOr(err, kErrSpin);
+            return;
+        }
+    }
+}
+
+__global__ void k_grid_empty(unsigned long long *p, int64_t n)
+{
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
+        p[i] = kGridEmpty;
+}
+
+size_t jacobi_grid_bytes() { return (size_t)(kGridSweeps - 1) * kGridRows * 8; }
+
 // Lanes per row: the smallest power of two (at most 64) not below the mean
 // row length divided by SP3MM_SPMV_ROW_DIV (default 4: about four entries
 // per lane, measured best on SA hierarchies of 7-point operators).
@@ -700,11 +828,45 @@ bool launch_jacobi_small(const int64_t *rp, const int32_t *col, const double *va
                          const double *b, double *x, double omega, int sweeps, int *err, size_t max_lds,
                          hipStream_t st)
 {
-    if (M <= 0 || M > kSmallRows || jacobi_small_lds(M, nnz) > max_lds) return false;
+    if (!jacobi_small_fits(M, nnz, max_lds)) return false;
     const int L = lanes_for(M, nnz);
     const size_t lds = jacobi_small_lds(M, nnz);
     SP3MM_BY_LANES(k_jacobi_small, dim3(1), dim3(1024), lds, st, rp, col, val, (int)M, (int)nnz, b, x, omega,
                    sweeps, err)
+    return true;
+}
+
+void launch_jacobi_zero(const int64_t *rp, const int32_t *col, const double *val, int64_t M, const double *b,
+                        double *xo, double omega, int *err, hipStream_t st)
+{
+    if (M > 0)
+        hipLaunchKernelGGL(k_jacobi_zero, dim3((unsigned)((M + 255) / 256)), dim3(256), 0, st, rp, col, val, M, b, xo,
+                           omega, err);
+}
+
+bool jacobi_small_fits(int64_t M, int64_t nnz, size_t max_lds)
+{
+    return M > 0 && M <= kSmallRows && jacobi_small_lds(M, nnz) <= max_lds;
+}
+
+// Launches nothing and returns false when a launch per sweep is as good: fewer
+// than kGridMin sweeps (clearing the buffers is a launch of its own), or rows
+// beyond what 256 workgroups hold.
+bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
+                        const double *b, double *x, void *buf, double omega, int sweeps, bool from_zero, int *err,
+                        hipStream_t st)
+{
+    constexpr int kGridMin = 4;
+    if (M <= 0 || M > kGridRows || sweeps < kGridMin || !buf) return false;
+    const int L = lanes_for(M, nnz);
+    auto *w = static_cast<unsigned long long *>(buf);
+    for (int k = 0; k < sweeps; k += kGridSweeps) {
+        const int n = std::min(kGridSweeps, sweeps - k);
+        if (n > 1) hipLaunchKernelGGL(k_grid_empty, dim3(grid1((n - 1) * M)), dim3(256), 0, st, w, (int64_t)(n - 1) * M);
+        const unsigned g = grid1(M, kGridThreads / L);
+        SP3MM_BY_LANES(k_jacobi_grid, dim3(g), dim3(kGridThreads), 0, st, rp, col, val, (int)M, b, x, w, omega, n,
+                       from_zero && k == 0, err)
+    }
     return true;
 }
 

@@ -39,14 +39,13 @@ void record_cycle(Context *c, VCycle &v, hipStream_t s)
         launch_spmv(M.rp, M.col, static_cast<const double *>(M.val), M.M, M.nnz, x, z, y, al, be, s);
     };
     for (int l = 0; l < v.nlev; l++) {
-        if (l > 0) launch_axpby(v.A[l].M, 0.0, nullptr, 0.0, v.x[l], s);  // a correction starts at zero
-        queue_jacobi(v.A[l], v.b[l], v.x[l], v.w[l], v.omega, v.nu1, err, s);
+        // a correction starts at zero
+        queue_jacobi(v.A[l], v.b[l], v.x[l], v.w[l], v.omega, v.nu1, err, s, l > 0);
         spmv_q(v.A[l], v.x[l], v.b[l], v.r[l], -1.0, 1.0);             // r = b - A x
         spmv_q(v.R[l], v.r[l], nullptr, v.b[l + 1], 1.0, 0.0);          // restrict
     }
     const int n = v.nlev;
-    launch_axpby(v.Ac.M, 0.0, nullptr, 0.0, v.x[n], s);
-    queue_jacobi(v.Ac, v.b[n], v.x[n], v.w[n], v.omega, v.csweeps, err, s);
+    queue_jacobi(v.Ac, v.b[n], v.x[n], v.w[n], v.omega, v.csweeps, err, s, true);
     for (int l = n - 1; l >= 0; l--) {
         spmv_q(v.P[l], v.x[l + 1], v.x[l], v.x[l], 1.0, 1.0);          // prolongate and correct
         queue_jacobi(v.A[l], v.b[l], v.x[l], v.w[l], v.omega, v.nu2, err, s);
