@@ -2515,7 +2515,8 @@ template <bool NUM, typename VT>
 __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A, SpOperand P,
                                                            const int32_t *__restrict__ rows,
                                                            const int *__restrict__ count, int cap, int slog1,
-                                                           int32_t *__restrict__ spill, int *__restrict__ nspill,
+                                                           int nxcd, int32_t *__restrict__ spill,
+                                                           int *__restrict__ nspill,
                                                            int32_t *__restrict__ rownnz,
                                                            const int64_t *__restrict__ crp,
                                                            int32_t *__restrict__ ccol, double *__restrict__ cval,
@@ -2538,7 +2539,8 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
     const int S = 1 << slog1;
     // list entries i index the per-row slots: at most cap_rows of them
     const int n = clamp_count(count, cap_rows, err);
-    for (int i = blockIdx.x; i < n; i += gridDim.x) {
+    const RowWalk walk = row_walk<1>(n, 0, nxcd);
+    for (int i = walk.i; i < walk.end; i += walk.stride) {
         const int r = rows[i];
         const int64_t e0 = R.rp[r], e1 = R.rp[r + 1];
         // window of the R*A row
@@ -2566,43 +2568,78 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
         if constexpr (NUM)
             for (int j = t; j < span1; j += kWin) V[j] = 0.0;
         __syncthreads();
-        // stage 1: sub-groups of S lanes per R entry walk its A row, four
-        // entries per lane at a time (their loads in flight together)
-        for (int64_t e = e0 + (t >> slog1); e < e1; e += (kWin >> slog1)) {
-            const int k = R.col[e];
-            double rv = 0.0;
-            if constexpr (NUM) rv = (double)rval[e];
-            const int a1 = A.rp32[k + 1];
-            for (int q0 = A.rp32[k] + (t & (S - 1)); q0 < a1; q0 += 4 * S) {
-                int jj[4];
-                double av[4];
+        // Stage 1: sub-groups of S lanes per R entry walk its A row, four
+        // entries per lane and step.  What bounds it is the latency of the
+        // loads, so a position past the row's end reads its last entry and is
+        // dropped afterwards: the four loads and the four bitmap reads carry no
+        // branch and are in flight together, and the next R entry's column is
+        // read during this one's row (a branch per load made each wait for the
+        // one before: 1728 rows of a 96^3 hierarchy 610 -> 567 us, 216 rows
+        // 316 -> 247 us; 2 or 8 entries per step are slower).
+        {
+            const int m = (int)(e1 - e0), step = kWin >> slog1;
+            int e = t >> slog1;
+            int k = e < m ? R.col[e0 + e] : 0;
+            while (e < m) {
+                const int a1 = A.rp32[k + 1];
+                int q0 = A.rp32[k] + (t & (S - 1));
+                double rv = 0.0;
+                if constexpr (NUM) rv = (double)rval[e0 + e];
+                e += step;
+                k = e < m ? R.col[e0 + e] : 0;
+                for (; q0 < a1; q0 += 4 * S) {
+                    int jj[4];
+                    double av[4];
+                    unsigned w[4];
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    const int q = q0 + u * S;
-                    const bool ok = q < a1;
-                    jj[u] = ok ? A.col[q] - lo1 : 0;
-                    av[u] = 0.0;
-                    if constexpr (NUM) av[u] = ok ? (double)aval[q] : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    if (q0 + u * S >= a1) break;
-                    const int j = jj[u];
-                    if ((unsigned)j >= (unsigned)span1) {  // an unsorted A row
-                        atomicOr(err, kErrBadInput);
-                        continue;
+                    for (int u = 0; u < 4; u++) {
+                        const int q = min(q0 + u * S, a1 - 1);
+                        jj[u] = A.col[q] - lo1;
+                        if constexpr (NUM) av[u] = (double)aval[q];
                     }
-                    const unsigned bit = 1u << (j & 31);
-                    if (!(B[j >> 5] & bit)) atomicOr(B + (j >> 5), bit);  // set bits are never cleared here
-                    if constexpr (NUM) atomicAdd(V + j, rv * av[u]);
+#pragma unroll
+                    for (int u = 0; u < 4; u++) w[u] = (unsigned)jj[u] < (unsigned)span1 ? B[jj[u] >> 5] : 0u;
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        if (q0 + u * S >= a1) break;
+                        const int j = jj[u];
+                        if ((unsigned)j >= (unsigned)span1) {  // an unsorted A row
+                            atomicOr(err, kErrBadInput);
+                            continue;
+                        }
+                        const unsigned bit = 1u << (j & 31);
+                        if (!(w[u] & bit)) atomicOr(B + (j >> 5), bit);  // set bits are never cleared here
+                        if constexpr (NUM) atomicAdd(V + j, rv * av[u]);
+                    }
                 }
+            }
+        }
+        __syncthreads();
+        // The present entries of the R*A row as a list of 16-bit positions at
+        // the end of the window area, so that no sub-group of stage 2 walks the
+        // absent ones (1728 rows of a 96^3 hierarchy: 1,100 entries in windows
+        // of 4,600 columns, 567 -> 455 us).  Without room for it, or with two
+        // thirds of the window present, positions are tested one by one.
+        static_assert(kWin * 32 >= 160 * 1024 / 8, "a lane per bitmap word");
+        long long present;
+        long long at = block_exclusive_scan(t < nw1 ? __popc(B[t]) : 0, lsh, present);
+        const int n1 = (int)present;
+        const int room = (2 * n1 + 7) / 8;  // the list's size in window values
+        bool listed = 3 * n1 < 2 * span1 && nw1 * 32 + room <= cap;
+        uint16_t *list = reinterpret_cast<uint16_t *>(V + (cap - room));
+        if (listed && t < nw1) {
+            unsigned x = B[t];
+            while (x) {
+                list[at++] = (uint16_t)(t * 32 + __ffs(x) - 1);
+                x &= x - 1;
             }
         }
         __syncthreads();
         // window of the forwarded row in P
         int lo2 = INT_MAX, hi2 = -1;
-        for (int j = t; j < span1; j += kWin) {
-            if (B[j >> 5] & (1u << (j & 31))) {
+        for (int jl = t; jl < (listed ? n1 : span1); jl += kWin) {
+            const int j = listed ? (int)list[jl] : jl;
+            if (listed || (B[j >> 5] & (1u << (j & 31)))) {
                 const int c = lo1 + j;
                 const int p0 = P.rp32[c], p1 = P.rp32[c + 1];
                 if (p1 > p0) {
@@ -2623,6 +2660,7 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
             }
             continue;
         }
+        if (off2 + nw2 * 32 + room > cap) listed = false;  // the list gives way to the values
         unsigned *B2 = B + nw1;
         double *V2 = V + off2;
         for (int w = t; w < nw2; w += kWin) B2[w] = 0u;
@@ -2631,15 +2669,17 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
         __syncthreads();
         // stage 2: sub-groups of kWinSub2 lanes walk the P rows of the present
         // entries (positions strided over the sub-groups), two entries per
-        // lane per step.  A lane per present entry walking its P row alone
+        // lane per step, loaded as in stage 1.  A lane per present entry walking its P row alone
         // made every load of a wavefront touch 64 rows (the 1728-row level
         // of a 96^3 hierarchy took 0.95 instead of 0.70 ms per product).
         double ps = 0.0;
         {
             constexpr int S2 = kWinSub2;
             const int sub = t & (S2 - 1), ngrp = kWin / S2;
-            for (int j = t / S2; j < span1; j += ngrp) {
-                if (!(B[j >> 5] & (1u << (j & 31)))) continue;
+            const int m = listed ? n1 : span1;
+            for (int jl = t / S2; jl < m; jl += ngrp) {
+                const int j = listed ? (int)list[jl] : jl;
+                if (!listed && !(B[j >> 5] & (1u << (j & 31)))) continue;
                 const int c = lo1 + j;
                 double x = 0.0;
                 if constexpr (NUM) x = V[j];
@@ -2647,13 +2687,15 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
                 for (int q0 = P.rp32[c] + sub; q0 < p1; q0 += 2 * S2) {
                     int jj[2];
                     double pv[2];
+                    unsigned w[2];
 #pragma unroll
                     for (int u = 0; u < 2; u++) {
-                        const bool ok = q0 + u * S2 < p1;
-                        jj[u] = ok ? P.col[q0 + u * S2] - lo2 : 0;
-                        pv[u] = 0.0;
-                        if constexpr (NUM) pv[u] = ok ? (double)pval[q0 + u * S2] : 0.0;
+                        const int q = min(q0 + u * S2, p1 - 1);
+                        jj[u] = P.col[q] - lo2;
+                        if constexpr (NUM) pv[u] = (double)pval[q];
                     }
+#pragma unroll
+                    for (int u = 0; u < 2; u++) w[u] = (unsigned)jj[u] < (unsigned)span2 ? B2[jj[u] >> 5] : 0u;
 #pragma unroll
                     for (int u = 0; u < 2; u++) {
                         if (q0 + u * S2 >= p1) break;
@@ -2663,7 +2705,7 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
                             continue;
                         }
                         const unsigned bit2 = 1u << (j2 & 31);
-                        if (!(B2[j2 >> 5] & bit2)) atomicOr(B2 + (j2 >> 5), bit2);
+                        if (!(w[u] & bit2)) atomicOr(B2 + (j2 >> 5), bit2);
                         if constexpr (NUM) {
                             const double pr = x * pv[u];
                             atomicAdd(V2 + j2, pr);
@@ -2760,7 +2802,11 @@ void launch_window_direct(bool num, int blocks, size_t lds, const SpOperand &R, 
     // workgroup (64 lanes each, 16 in flight, made the 1728-row level of a
     // 96^3 hierarchy 6% slower)
     if (slog1 > 4) slog1 = 4;
-#define SP3MM_WIN_ARGS R, A, P, rows, count, cap, slog1, spill, nspill, rownnz, crp, ccol, cval, rowsum, out_cap, \
+    // neighbouring rows on one XCD's L2 (1728 rows of a 96^3 hierarchy: 400 -> 124
+    // MB fetched per product); a grid that is no multiple of the XCDs has a row
+    // per workgroup and needs every one of them
+    const int nxcd = blocks % kXcds == 0 ? kXcds : 1;
+#define SP3MM_WIN_ARGS R, A, P, rows, count, cap, slog1, nxcd, spill, nspill, rownnz, crp, ccol, cval, rowsum, out_cap, \
                        err, slotn, scol, sval, cap_rows
     if (f32in) {
         if (num) hipLaunchKernelGGL((k_window_direct<true, float>), dim3(blocks), dim3(kWin), bytes, st, SP3MM_WIN_ARGS);
