@@ -1287,7 +1287,7 @@ struct FusedPlan {
         return likely_bin(thr, R, A);
     }
 
-    void launch_main(Context *c, hipStream_t s, int i, bool early = false)
+    void launch_main(Context *c, hipStream_t s, int i, bool early = false, bool in_place = false)
     {
         const FusedCfg &f = cfg[i];
         const int64_t M = R.M;
@@ -1313,8 +1313,9 @@ struct FusedPlan {
                                 fix.as<int32_t>() + nbase[i], d()->counts2 + i, &d()->err, max_blocks(c), s, tu);
         else
             launch_direct_fused(f.G, f.H1, f.H2, slog1, slog2, r(), a(), p(), lists.as<int32_t>() + (int64_t)i * M,
-                                count, slot_rows(i), rown.as<int32_t>(), slot_n(i), slot_col(i), slot_val(i),
-                                retry.as<int32_t>(), &d()->nretry, &d()->err, max_blocks(c), s, f32, t);
+                                count, slot_rows(i), rown.as<int32_t>(), slot_n(i), in_place ? C.col : slot_col(i),
+                                in_place ? static_cast<double *>(C.val) : slot_val(i), retry.as<int32_t>(),
+                                &d()->nretry, &d()->err, max_blocks(c), s, f32, t, in_place ? C.rp : nullptr);
     }
 
     // export_ctl: the first gather also copies the control block to the host
@@ -1870,6 +1871,30 @@ struct FusedPlan {
                          &want);
     }
 
+    // A replay on operands whose patterns are those of build(): the lists,
+    // populations and offsets of build() hold, so only the values are
+    // recomputed, straight into the output.  Binning, scan, gather and the
+    // check of the sizes are left out (8 launches of 5 us and 24 us of gather
+    // for the finest product of a 96^3 hierarchy).  Not for plans with retried,
+    // spilled or scattered rows, which need their lists and slots.  The caller
+    // clears the error word.
+    bool fixed_ok() const
+    {
+        bool plain = built && !mixed && !f32 && nretry == 0 && nspill == 0 && !(lscatter && nlong > 0);
+        for (int i = 0; i < thr.nb; i++) plain = plain && !(cnt[i] > 0 && cfg[i].scatter);
+        return plain;
+    }
+    void record_fixed(Context *c, hipStream_t s)
+    {
+        for (int i = 0; i < thr.nb; i++)
+            if (cnt[i]) launch_main(c, s, i, false, true);
+        if (nlong > 0)
+            launch_window_direct(true, std::min(nlong, c->num_cu), c->max_lds - 1024, r(), a(), p(),
+                                 lists.as<int32_t>() + (int64_t)thr.nb * R.M, d()->counts + thr.nb, dlog1,
+                                 spill.as<int32_t>(), &d()->nspill, nullptr, C.rp, C.col,
+                                 static_cast<double *>(C.val), nullptr, ccap, &d()->err, s, f32);
+    }
+
     // after a replay: did the device see the sizes this plan was built for?
     int check(Context *c)
     {
@@ -2188,8 +2213,9 @@ struct SaPlan {
 // P = (I - omega D^-1 A) P0 from A's rows and the aggregate ids (k_sa_rows).
 // build() finds the row lengths and fills P, allocated for the most entries
 // it can have (A's and a diagonal per row), and with `replayable` also the
-// longest row (atomics: 75 us on 10^5 rows); record() refills its columns and
-// values for new values of A (same pattern), without host synchronisation.
+// longest row (atomics: 75 us on 10^5 rows); fill() refills its columns and
+// values for new values of A (same pattern), without host synchronisation, and
+// leaves clearing the error word to the caller.
 // build() returns 1, nothing allocated, when a row of A is longer than the
 // kernel takes (the caller forms S and S P0 instead).
 struct SaRowsPlan {
@@ -2250,11 +2276,6 @@ struct SaRowsPlan {
                        mode, P.rp, nullptr, P.col, static_cast<double *>(P.val), nullptr, longest, &d()->err, s);
     }
 
-    void record(Context *, hipStream_t s)
-    {
-        launch_fill_i32(&d()->err, 1, 0, s);
-        fill(s);
-    }
 };
 
 int sa_prolongator(const sp3mm_dmat &A, const int64_t *agg, int64_t nagg, double omega, int mode, sp3mm_dmat &P)
@@ -3297,16 +3318,24 @@ struct HierLevel {
     FusedPlan rap;      // A_{l+1} = R * A_l * P
     const sp3mm_dmat &P() const { return by_rows ? rows.P : pplan.C; }
 
+    // the caller has cleared the error words
     void record(Context *c, hipStream_t s)
     {
         if (by_rows) {
-            rows.record(c, s);
+            rows.fill(s);
         } else {
             sa.record(c, s);
-            pplan.record(c, s);
+            replay(pplan, c, s);
         }
         tr.record(c, s);
-        rap.record(c, s);
+        // A_l, P and R have the patterns of build(): A_0's is checked by its
+        // fingerprint, and the others follow from it and the aggregates
+        replay(rap, c, s);
+    }
+    static void replay(FusedPlan &p, Context *c, hipStream_t s)
+    {
+        if (p.fixed_ok()) p.record_fixed(c, s);
+        else p.record(c, s);
     }
     void release_all()
     {
@@ -3329,6 +3358,12 @@ struct Hier {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     double ms_build = 0;
+
+    void record(Context *c, hipStream_t s)
+    {
+        launch_clear_words(errp.as<int *>(), nerr, s);
+        for (auto &l : lv) l->record(c, s);
+    }
 };
 
 static int pattern_fingerprint(Context *c, const sp3mm_dmat &A, Buf &buf, unsigned long long &out)
@@ -3492,7 +3527,7 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
             (void)hipGetLastError();
             return h;  // usable without a graph
         }
-        for (auto &l : h->lv) l->record(c, s);
+        h->record(c, s);
         if (hipStreamEndCapture(s, &h->graph) != hipSuccess ||
             hipGraphInstantiate(&h->exec, h->graph, nullptr, nullptr, 0) != hipSuccess) {
             (void)hipGetLastError();
@@ -3525,8 +3560,7 @@ int hier_update(void *hp, bool use_graph, double *ms)
     SP3MM_HIP(hipEventCreate(&e1));
     SP3MM_HIP(hipEventRecord(e0, c->stream));
     if (use_graph) SP3MM_HIP(hipGraphLaunch(h->exec, c->stream));
-    else
-        for (auto &l : h->lv) l->record(c, c->stream);
+    else h->record(c, c->stream);
     SP3MM_HIP(hipEventRecord(e1, c->stream));
     launch_or_words(h->errp.as<const int *>(), h->nerr, h->errs.as<int>(), c->stream);
     SP3MM_HIP(hipMemcpyAsync(c->host_small, h->errs.p, 4, hipMemcpyDeviceToHost, c->stream));

@@ -155,7 +155,7 @@ void launch_direct_fused(int G, int H1, int H2, int slog1, int slog2, const SpOp
                          const SpOperand &P, const int32_t *rows, const int *count, int rows_host,
                          int32_t *rownnz, int32_t *slotn, int32_t *scol, double *sval, int32_t *retry,
                          int *nretry, int *err, int max_blocks, hipStream_t st, bool f32in,
-                         const Tuning &tu);
+                         const Tuning &tu, const int64_t *place = nullptr);
 // What k_sample_rows learns from kSampleRows rows of R: per bin of the row
 // bound the number of rows sampled and the most distinct stage-1 and stage-2
 // keys of any of them (INT32_MAX: more than the kernel counts), and per stage
@@ -257,6 +257,8 @@ void launch_fingerprint(const int64_t *rp, int64_t M, const int32_t *col, int64_
                         hipStream_t st);
 // *out = OR of the n device words *words[i] (one wavefront)
 void launch_or_words(const int *const *words, int n, int *out, hipStream_t st);
+// *words[i] = 0 for all i
+void launch_clear_words(int *const *words, int n, hipStream_t st);
 // setup.hip: transpose and smoothed-aggregation prolongator
 void launch_col_count(const int32_t *col, int64_t nnz, int32_t *cnt, hipStream_t st);
 void launch_transpose_scatter(const int64_t *rp, const int32_t *col, const void *val, bool f32, int64_t M,

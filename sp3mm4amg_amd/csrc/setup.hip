@@ -932,4 +932,16 @@ void launch_or_words(const int *const *words, int n, int *out, hipStream_t st)
     hipLaunchKernelGGL(k_or_words, dim3(1), dim3(64), 0, st, words, n, out);
 }
 
+// every plan's error word, cleared by one launch (a launch per word costs 4.6
+// us each in a replay)
+__global__ void k_clear_words(int *const *words, int n)
+{
+    for (int i = threadIdx.x; i < n; i += blockDim.x) *words[i] = 0;
+}
+
+void launch_clear_words(int *const *words, int n, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_clear_words, dim3(1), dim3(64), 0, st, words, n);
+}
+
 }  // namespace sp3mm
