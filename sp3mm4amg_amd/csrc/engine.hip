@@ -3368,9 +3368,13 @@ struct Hier {
 
 static int pattern_fingerprint(Context *c, const sp3mm_dmat &A, Buf &buf, unsigned long long &out)
 {
-    launch_fingerprint(A.rp, A.M, A.col, A.nnz, buf.as<unsigned long long>(), c->stream);
-    SP3MM_HIP(hipMemcpyAsync(c->host_small, buf.p, 8, hipMemcpyDeviceToHost, c->stream));
-    SP3MM_HIP(hipStreamSynchronize(c->stream));
+    auto *state = buf.as<unsigned long long>();
+    void *dst = c->host_small_dev;
+    launch_fingerprint(A.rp, A.M, A.col, A.nnz, state, dst ? static_cast<unsigned long long *>(dst) : state + 2,
+                       c->stream);
+    SP3MM_HIP(hipGetLastError());
+    if (!dst) SP3MM_HIP(hipMemcpyAsync(c->host_small, state + 2, 8, hipMemcpyDeviceToHost, c->stream));
+    SP3MM_HIP(spin_stream(c->stream));
     memcpy(&out, c->host_small, 8);
     return 0;
 }
@@ -3420,13 +3424,14 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
     Hier *h = new Hier();
     h->A0 = A;
     h->A0.owned = 0;
-    h->fpbuf = Buf(8);
+    h->fpbuf = Buf(24);  // the fingerprint kernel's two words of state, and its result
     Buf ctl(sizeof(Ctl));
     if (!h->fpbuf.p || !ctl.p) {
         set_error("hierarchy: allocation failed");
         delete h;
         return nullptr;
     }
+    launch_fill_i32(h->fpbuf.as<int32_t>(), 4, 0, c->stream);
     Timer tm(c->stream, true);
     const int e0 = tm.mark();
     if (pattern_fingerprint(c, A, h->fpbuf, h->fp)) {
@@ -3555,23 +3560,19 @@ int hier_update(void *hp, bool use_graph, double *ms)
         set_error("hierarchy: the pattern of A changed since the hierarchy was built (only values may change)");
         return -1;
     }
-    hipEvent_t e0, e1;
-    SP3MM_HIP(hipEventCreate(&e0));
-    SP3MM_HIP(hipEventCreate(&e1));
-    SP3MM_HIP(hipEventRecord(e0, c->stream));
+    Timer tm(c->stream, true);
+    const int e0 = tm.mark();
     if (use_graph) SP3MM_HIP(hipGraphLaunch(h->exec, c->stream));
     else h->record(c, c->stream);
-    SP3MM_HIP(hipEventRecord(e1, c->stream));
-    launch_or_words(h->errp.as<const int *>(), h->nerr, h->errs.as<int>(), c->stream);
-    SP3MM_HIP(hipMemcpyAsync(c->host_small, h->errs.p, 4, hipMemcpyDeviceToHost, c->stream));
-    SP3MM_HIP(hipStreamSynchronize(c->stream));
+    const int e1 = tm.mark();
+    void *dst = c->host_small_dev;
+    launch_or_words(h->errp.as<const int *>(), h->nerr, dst ? static_cast<int *>(dst) : h->errs.as<int>(), c->stream);
+    SP3MM_HIP(hipGetLastError());
+    if (!dst) SP3MM_HIP(hipMemcpyAsync(c->host_small, h->errs.p, 4, hipMemcpyDeviceToHost, c->stream));
+    SP3MM_HIP(spin_stream(c->stream));
     int err = 0;
     memcpy(&err, c->host_small, 4);
-    float t = 0.f;
-    (void)hipEventElapsedTime(&t, e0, e1);
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    if (ms) *ms = t;
+    if (ms) *ms = tm.ms(e0, e1);
     if (err) {
         set_error("hierarchy update: %s", err_text(err));
         return -1;

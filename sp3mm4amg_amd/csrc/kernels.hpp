@@ -252,9 +252,10 @@ void launch_rp_shift(const int64_t *rp, int64_t n, int base, int64_t *out, hipSt
 void launch_f64_to_f32(const double *in, int64_t n, float *out, hipStream_t st);
 void launch_f32_to_f64(const float *in, int64_t n, double *out, hipStream_t st);
 void launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t st);
-// order-sensitive 64-bit fingerprint of a CSR pattern (offsets and columns) into *out
+// order-sensitive 64-bit fingerprint of a CSR pattern (offsets and columns)
+// into *dst; out: two words of state, zero before and after
 void launch_fingerprint(const int64_t *rp, int64_t M, const int32_t *col, int64_t nnz, unsigned long long *out,
-                        hipStream_t st);
+                        unsigned long long *dst, hipStream_t st);
 // *out = OR of the n device words *words[i] (one wavefront)
 void launch_or_words(const int *const *words, int n, int *out, hipStream_t st);
 // *words[i] = 0 for all i

@@ -2,6 +2,8 @@
 (several bins, long rows in LDS windows), and the full replay that plans with
 retried rows keep.  Each replay against a hierarchy built call by call from the
 same values."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -47,3 +49,26 @@ def test_replays_match_fresh_builds(dims, levels, tuning):
         dA.free()
     finally:
         L.set_tuning(None)
+
+
+@pytest.mark.parametrize("dims", [(4, 3, 2), (16, 16, 4), (64, 61, 59)])
+def test_fingerprint_sees_the_last_row(dims):
+    """Patterns of one workgroup's work up to many steps of its loop: a column
+    of the last row moved by one is refused, and moved back accepted."""
+    L.init(0)
+    A = problems.poisson_operator(dims)
+    agg, d = problems.structured_aggregation(dims, (2, 2, 2))
+    dA = L.DeviceCSR.upload(A)
+    H = L.Hierarchy(dA, [(agg, int(np.prod(d)))], graph=True)
+    at = int(A.irp[-2])
+    addr = C.cast(dA.d.col, C.c_void_p).value + 4 * at
+    for shift, ok in ((1, False), (0, True)):
+        col = np.array([A.ja[at] - shift], np.int32)
+        assert L.lib().sp3mm_copy_to_device(addr, col.ctypes.data, 4) == 0
+        if ok:
+            H.update()
+        else:
+            with pytest.raises(RuntimeError, match="pattern"):
+                H.update()
+    H.free()
+    dA.free()
