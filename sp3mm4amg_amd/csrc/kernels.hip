@@ -3294,6 +3294,18 @@ __global__ void k_extract(const int64_t *__restrict__ rp, const int32_t *__restr
     }
 }
 
+// dst[i] = rp[at[i]], i < n: the entry ranges of a batch's products to pinned
+// host memory, once per run instead of two copies and their waits per result
+__global__ void k_pick_offsets(const int64_t *__restrict__ rp, const int64_t *__restrict__ at, int n, int64_t *dst)
+{
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) dst[i] = rp[at[i]];
+}
+
+void launch_pick_offsets(const int64_t *rp, const int64_t *at, int n, int64_t *dst, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_pick_offsets, dim3((unsigned)std::min((n + 255) / 256, 256)), dim3(256), 0, st, rp, at, n, dst);
+}
+
 void launch_extract(const int64_t *rp, const int32_t *col, const double *val, int64_t r0, int64_t M, int32_t coloff,
                     int64_t *orp, int32_t *orp32, int32_t *ocol, double *oval, hipStream_t st)
 {

@@ -236,6 +236,7 @@ struct PackItem {
     int32_t pad;
 };
 void launch_pack(const PackItem *items, int count, int vtype, int64_t *rp, int32_t *col, void *val, hipStream_t st);
+void launch_pick_offsets(const int64_t *rp, const int64_t *at, int n, int64_t *dst, hipStream_t st);
 void launch_extract(const int64_t *rp, const int32_t *col, const double *val, int64_t r0, int64_t M, int32_t coloff,
                     int64_t *orp, int32_t *orp32, int32_t *ocol, double *oval, hipStream_t st);
 
