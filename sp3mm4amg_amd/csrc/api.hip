@@ -51,6 +51,47 @@ int sp3mm_sync(void)
     return consumer_wait(c);
 }
 
+static void set_not_csr(int base)
+{
+    set_error("upload: matrix is not valid sorted CSR (offsets must be monotone from %d to "
+              "nnz+%d, columns in [%d, N+%d) and strictly increasing inside each row)",
+              base, base, base, base);
+}
+
+// sp3mm_dmat_upload for arrays that host_upload takes: 0 or -1, or 1 when it
+// has not taken them after all
+static int upload_large(sp3mm_dmat *out, int64_t M, int64_t N, int64_t nnz, const int64_t *irp, const int64_t *ja,
+                        const void *val, int vtype, int base)
+{
+    Context *c = ctx();
+    if (!c) return -1;
+    std::lock_guard<std::recursive_mutex> lk(c->mu);
+    hipStream_t s = c->stream;
+    sp3mm_dmat m;
+    Buf err(64);
+    if (!err.p || !c->host_small_dev) return 1;
+    if (dmat_alloc(m, M, N, nnz, vtype)) return -1;
+    HostCheck chk;
+    int rc = host_upload(c, m, irp, ja, val, base, chk);
+    if (rc == 0) {
+        launch_fill_i32(err.as<int32_t>(), 1, 0, s);
+        // offsets that decrease bound no row: nothing on the device reads them
+        if (chk.bad_row < 0) launch_csr_finish(m.rp32, m.col, M, m.rp, err.as<int>(), s);
+        launch_export_words(err.p, c->host_small_dev, 1, s);
+        hipError_t e = hipGetLastError();
+        if (e == hipSuccess) e = spin_stream(s);
+        int herr = 0;
+        memcpy(&herr, c->host_small, 4);
+        if (e != hipSuccess) set_error("upload: HIP error %s", hipGetErrorString(e));
+        else if (chk.bad_row >= 0) set_error("upload: row offsets decrease at row %lld", (long long)chk.bad_row);
+        else if (chk.bad_col || herr) set_not_csr(base);
+        if (e != hipSuccess || chk.bad_row >= 0 || chk.bad_col || herr) rc = -1;
+    }
+    if (rc) dmat_release(m);
+    else *out = m;
+    return rc;
+}
+
 int sp3mm_dmat_upload(sp3mm_dmat *out, int64_t M, int64_t N, int64_t nnz, const int64_t *irp,
                       const int64_t *ja, const void *val, int32_t vtype, int32_t base)
 {
@@ -74,6 +115,10 @@ int sp3mm_dmat_upload(sp3mm_dmat *out, int64_t M, int64_t N, int64_t nnz, const 
         set_error("upload: row offsets must run from %d to nnz+%d (got %lld .. %lld, nnz %lld)", base, base,
                   (long long)irp[0], (long long)irp[M], (long long)nnz);
         return -1;
+    }
+    if (host_io_fits(M, nnz, vtype)) {
+        const int rc = upload_large(out, M, N, nnz, irp, ja, val, vtype, base);
+        if (rc <= 0) return rc;
     }
     for (int64_t r = 0; r < M; r++) {
         if (irp[r + 1] < irp[r]) {
@@ -115,9 +160,7 @@ int sp3mm_dmat_upload(sp3mm_dmat *out, int64_t M, int64_t N, int64_t nnz, const 
         if (hipMemcpyAsync(&herr, err.p, 4, hipMemcpyDeviceToHost, s) != hipSuccess) { rc = -1; break; }
         if (hipStreamSynchronize(s) != hipSuccess) { rc = -1; break; }
         if (herr) {
-            set_error("upload: matrix is not valid sorted CSR (offsets must be monotone from %d to "
-                      "nnz+%d, columns in [%d, N+%d) and strictly increasing inside each row)",
-                      base, base, base, base);
+            set_not_csr(base);
             rc = -2;
         }
     } while (0);
@@ -228,6 +271,10 @@ int sp3mm_dmat_download(const sp3mm_dmat *m, int64_t *irp, int64_t *ja, void *va
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     hipStream_t s = c->stream;
     const int64_t M = m->M, nnz = m->nnz;
+    if (ja && val && host_io_fits(M, nnz, m->vtype)) {
+        const int rc = host_download(c, *m, irp, ja, val, base);
+        if (rc <= 0) return rc;
+    }
     Buf trp((size_t)(M + 1) * 8), tja((size_t)(nnz ? nnz : 1) * 8);
     if (!trp.p || !tja.p) {
         set_error("download: staging allocation failed");

@@ -43,6 +43,14 @@ class Pool {
     std::mutex mu_;
 };
 
+// Pinned staging of large host copies (16 MB, allocated by the first one), and
+// an event per group of slots.
+struct HostRing {
+    unsigned char *mem = nullptr;
+    unsigned char *dev = nullptr;  // its device-side address
+    std::vector<hipEvent_t> ev;
+};
+
 struct Context {
     int device = -1;
     hipStream_t stream = nullptr;      // the stream every call is queued on
@@ -74,6 +82,7 @@ struct Context {
     // state of the level consumers (SpMV, Jacobi, dot): a dot result, a sticky
     // error word set by Jacobi sweeps, and the dot's partial sums
     void *cons = nullptr;
+    HostRing *ring = nullptr;  // used under mu, idle outside a copy
     std::recursive_mutex mu;
 };
 
@@ -87,6 +96,21 @@ struct ConsState {
     int pad;
 };
 ConsState *cons_state(Context *c);
+
+// Large host arrays to a device matrix (m allocated, nnz < 2^31) and back,
+// through pinned staging and host threads: 0 done, 1 not taken (no threads or
+// no pinned memory: the caller copies them itself), -1 failed.  An upload
+// leaves m.rp32, m.col and m.val queued on the stream; what it found wrong with
+// the arrays is in `chk`, and m.rp and the order of the columns inside a row
+// are left to the caller (launch_csr_finish).
+struct HostCheck {
+    int64_t bad_row = -1;  // first row whose offsets decrease
+    bool bad_col = false;  // a column out of range
+};
+bool host_io_fits(int64_t M, int64_t nnz, int vtype);
+int host_upload(Context *c, const sp3mm_dmat &m, const int64_t *irp, const int64_t *ja, const void *val, int base,
+                HostCheck &chk);
+int host_download(Context *c, const sp3mm_dmat &m, int64_t *irp, int64_t *ja, void *val, int base);
 
 // Waits for the library stream and reports (and clears) an error that a
 // stream-ordered consumer call left in the device error word.

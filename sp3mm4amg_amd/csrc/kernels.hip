@@ -2242,6 +2242,23 @@ __global__ void k_col_convert(const int64_t *__restrict__ in, const int64_t *__r
     if (bad) atomicOr(err, kErrBadInput);
 }
 
+// 64-bit offsets from the 32-bit ones, and the check that columns increase
+// inside each row; 8 lanes per row, so that neighbouring lanes read neighbouring
+// columns
+__global__ void k_csr_finish(const int32_t *__restrict__ rp32, const int32_t *__restrict__ col, int64_t M,
+                             int64_t *__restrict__ rp, int *__restrict__ err)
+{
+    const int64_t r = (int64_t)blockIdx.x * (blockDim.x / 8) + threadIdx.x / 8;
+    if (r > M) return;
+    const int e0 = rp32[r];
+    if (threadIdx.x % 8 == 0) rp[r] = e0;
+    if (r == M) return;
+    const int e1 = rp32[r + 1];
+    bool bad = false;
+    for (int e = e0 + threadIdx.x % 8; e + 1 < e1; e += 8) bad |= col[e] >= col[e + 1];
+    if (bad) atomicOr(err, kErrBadInput);
+}
+
 __global__ void k_col_widen(const int32_t *__restrict__ col, int64_t nnz, int base, int64_t *__restrict__ out)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3344,6 +3361,11 @@ void launch_col_convert(const int64_t *in, const int64_t *rp, int64_t M, int64_t
     if (M == 0) return;
     hipLaunchKernelGGL(k_col_convert, dim3(blocks_for(M, 256)), dim3(256), 0, st, in, rp, M, N, base, col,
                        err);
+}
+
+void launch_csr_finish(const int32_t *rp32, const int32_t *col, int64_t M, int64_t *rp, int *err, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_csr_finish, dim3(blocks_for(M + 1, 32)), dim3(256), 0, st, rp32, col, M, rp, err);
 }
 
 void launch_col_widen(const int32_t *col, int64_t nnz, int base, int64_t *out, hipStream_t st)

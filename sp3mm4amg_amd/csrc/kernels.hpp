@@ -248,6 +248,8 @@ void launch_rp_convert(const int64_t *in, int64_t M, int64_t nnz, int base, int6
                        int *err, hipStream_t st);
 void launch_col_convert(const int64_t *in, const int64_t *rp, int64_t M, int64_t N, int base, int32_t *col,
                         int *err, hipStream_t st);
+// rp from rp32 (valid offsets), and columns of a row not increasing -> *err
+void launch_csr_finish(const int32_t *rp32, const int32_t *col, int64_t M, int64_t *rp, int *err, hipStream_t st);
 void launch_col_widen(const int32_t *col, int64_t nnz, int base, int64_t *out, hipStream_t st);
 void launch_rp_shift(const int64_t *rp, int64_t n, int base, int64_t *out, hipStream_t st);
 void launch_f64_to_f32(const double *in, int64_t n, float *out, hipStream_t st);
