@@ -190,6 +190,10 @@ int init_device(int dev)
             (void)hipGetLastError();
             c->board = nullptr;
         }
+        if (hipMalloc((void **)&c->ticket, 64) != hipSuccess || hipMemset(c->ticket, 0, 64) != hipSuccess) {
+            (void)hipGetLastError();
+            c->ticket = nullptr;
+        }
     }
     // this device's copy of the fixed scratch array (sp3mm_rap_noalloc reports
     // an error if it cannot be resolved; the other entry points do not use it)
@@ -1431,6 +1435,17 @@ struct FusedPlan {
                       reassoc_possible(c), one ? &ob : nullptr, R.M > 0 && R.nnz >= (int64_t)kWaveUbRow * R.M);
     }
 
+    // the one-bin test by itself, its answer to the host (see k_one_bin)
+    void queue_one_bin(Context *c, hipStream_t s, unsigned long long seq)
+    {
+        const int3 set = make_int3((int)(offsetof(Ctl, counts) / 4) + pred, (int)(offsetof(Ctl, rawc) / 4) + pred,
+                                   (int)(offsetof(Ctl, pred_count) / 4));
+        launch_one_bin(r(), a(), thr.v[pred], mlen.as<int>(), c->ticket, lists.as<int32_t>() + (int64_t)pred * R.M,
+                       d(), (int)(sizeof(Ctl) / 4), set, (int)(offsetof(Ctl, onebin) / 4),
+                       reinterpret_cast<unsigned *>(c->poll_dev),
+                       reinterpret_cast<unsigned long long *>(c->poll_dev + kPollFlagOff), seq, s);
+    }
+
     // R*(A*P) instead of the direct forwarding: when at least half of R's
     // rows are long rows or rows of the multi-wavefront bins, at least half
     // of R's rows are unstructured (their columns spread over more than a
@@ -1660,9 +1675,14 @@ struct FusedPlan {
             may_sample && (pred >= 0 || (scatter_fits(c) && (double)R.nnz * ((double)A.nnz / (double)A.M) <=
                                                                 kScatterMerge * (double)R.M * (double)A.N));
         const unsigned long long sseq = sampling ? queue_sample(c, nullptr, nullptr, pred) : 0;
-        const unsigned long long seq = c->poll_host ? ++c->poll_seq : 0;
-        launch_binning(c, s, seq);
-        const int eu = mk(tm);
+        // A product whose rows may all fit the likely bin asks for that first; the
+        // likely bin's launch behind it goes on or ends at once, and the host
+        // queues the binning only if it has to.  (Plans to be replayed bin on
+        // the device every time.)
+        bool one = onebin_ok && !keep && c->poll_host && c->ticket;
+        unsigned long long seq = c->poll_host ? ++c->poll_seq : 0;
+        if (one) queue_one_bin(c, s, seq);
+        else launch_binning(c, s, seq);
         retry = Buf((size_t)(M ? M : 1) * 4);
         slotn = Buf((size_t)(M ? M : 1) * 4);
         fix = Buf((size_t)(M ? M : 1) * 4);
@@ -1672,6 +1692,7 @@ struct FusedPlan {
             set_error("scratch allocation failed");
             return -1;
         }
+        const int eu = mk(tm);
         // the binning runs while the sample arrives
         if (sampling) {
             SampleOut so;
@@ -1700,7 +1721,25 @@ struct FusedPlan {
             en0 = mk(tm);
             launch_main(c, s, own, true);
         }
-        if (wait_ctl(c, d(), seq, h)) return -1;
+        if (one) {
+            if (wait_flag(c, kPollFlagOff, seq)) return -1;
+            unsigned fits = 0;
+            memcpy(&fits, c->poll_host, sizeof fits);
+            one = fits != 0;
+            if (!one) {
+                onebin_ok = false;
+                seq = ++c->poll_seq;
+                launch_binning(c, s, seq);
+                if (own >= 0) launch_main(c, s, own, true);
+            }
+        }
+        if (one) {  // what k_one_bin left in the control block
+            memset(&h, 0, sizeof h);
+            h.counts[pred] = h.rawc[pred] = h.pred_count = (int)M;
+            h.onebin = 1;
+        } else if (wait_ctl(c, d(), seq, h)) {
+            return -1;
+        }
         onebin = h.onebin != 0;
         mac1 = onebin ? -1 : (long long)h.totals[0];  // one-bin mode: the bounds were not summed
         wide = h.totals[2];
@@ -1770,15 +1809,25 @@ struct FusedPlan {
         } else if (dmat_alloc(C, M, P.N, 0, SP3MM_F64)) {
             return -1;
         }
-        launch_scan(rown.as<int32_t>(), M, C.rp, C.rp32, tiles.as<long long>(), &d()->nnz, s);
+        // rows in one bin sit in its slots in row order
+        const bool joint = speculate && onebin && own >= 0 && own == pred && !ext_out && c->host_small_dev &&
+                           scan_gather_fits(M);
+        if (!joint) launch_scan(rown.as<int32_t>(), M, C.rp, C.rp32, tiles.as<long long>(), &d()->nnz, s);
         if (speculate) {
             if (ext_out)
                 ccap = ext_cap;  // the caller's arrays; a product that outgrows them is caught below
             else if (alloc_out(c, stot))
                 return -1;
-            spec = true;
-            const bool early = launch_tail(c, s, true);
-            spec = false;
+            bool early = joint;
+            if (joint) {
+                launch_scan_gather(rown.as<int32_t>(), M, C.rp, C.rp32, tiles.as<long long>(), &d()->nnz, slot_n(own),
+                                   cfg[own].H2, slot_col(own), slot_val(own), C.col, static_cast<double *>(C.val),
+                                   ccap, &d()->err, d(), c->host_small_dev, (int)(sizeof(Ctl) / 4), s);
+            } else {
+                spec = true;
+                early = launch_tail(c, s, true);
+                spec = false;
+            }
             defer_retry = false;
             if (early) {
                 // the control block is in the host mirror once the stream ends

@@ -64,6 +64,7 @@ struct Context {
     // no schedule was set: large products take their table sizes and hash
     // multipliers from a sample of their rows (FusedPlan::adapt)
     bool adapt = true;
+    int *ticket = nullptr;  // device word of launch_one_bin, zero between launches (null: not available)
     SampleBoard *board = nullptr;  // device scratch of the sampling (null: not available)
     // device address of the fixed scratch array of the allocation-free entry
     // point on this device (null if it could not be resolved)

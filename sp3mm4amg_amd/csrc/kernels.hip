@@ -138,6 +138,100 @@ __global__ void __launch_bounds__(256) k_row_maxlen(const IA *__restrict__ arp, 
     }
 }
 
+// One-bin mode in one launch, for plans whose host can still choose: the longest
+// rows as in k_row_maxlen; the last workgroup decides, writes the control block
+// that the binning would have left when every row fits the bin (`words` words,
+// those of `set` the row count, `one_word` 1; all 0 otherwise, which ends the main
+// kernel queued behind this one at once), and tells the host.  The list of the
+// bin is every row in order.  Replaces four launches of 3 to 5 us each, two
+// thirds of what a small product runs before its main kernel.
+// 64 workgroups: one addition each to the ticket, at 15 ns (state[0]; zero
+// before and after), and 1024 lanes with four rows in flight.
+constexpr int kOneBinBlocks = 64, kOneBinThreads = 1024;
+static_assert(kOneBinBlocks <= kMaxLenBlocks && kOneBinBlocks <= kOneBinThreads, "a partial per lane");
+template <typename IA, typename IB>
+__global__ void __launch_bounds__(kOneBinThreads) k_one_bin(const IA *__restrict__ arp, int64_t M,
+                                                            const IB *__restrict__ brp, int64_t BM, long long bound,
+                                                            int *__restrict__ part, int *state, int32_t *list,
+                                                            uint32_t *ctl, int words, int3 set, int one_word,
+                                                            unsigned *host, unsigned long long *flag,
+                                                            unsigned long long seq)
+{
+    __shared__ int red[2][kOneBinThreads / 64];
+    __shared__ bool last;
+    const int t = threadIdx.x;
+    const int64_t stride = (int64_t)gridDim.x * kOneBinThreads, i0 = (int64_t)blockIdx.x * kOneBinThreads + t;
+    auto longest = [&](const auto *rp, int64_t n) {
+        int64_t m = 0;
+        for (int64_t i = i0; i < n; i += 4 * stride) {
+            int64_t d[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int64_t k = i + u * stride;
+                d[u] = k < n ? (int64_t)(rp[k + 1] - rp[k]) : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) m = max(m, d[u]);
+        }
+        return (int)min(m, (int64_t)INT32_MAX);
+    };
+    auto reduce = [&](int &a, int &b) {
+        for (int o = 32; o > 0; o >>= 1) {
+            a = max(a, __shfl_xor(a, o));
+            b = max(b, __shfl_xor(b, o));
+        }
+        if (lane() == 0) {
+            red[0][t / 64] = a;
+            red[1][t / 64] = b;
+        }
+        __syncthreads();
+        for (int w = 0; w < kOneBinThreads / 64; w++) {
+            a = max(a, red[0][w]);
+            b = max(b, red[1][w]);
+        }
+        __syncthreads();
+    };
+    int ma = longest(arp, M), mb = longest(brp, BM);
+    for (int64_t i = i0; i < M; i += stride) list[i] = (int32_t)i;
+    reduce(ma, mb);
+    if (t == 0) {
+        __hip_atomic_store(part + 2 * blockIdx.x, ma, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(part + 2 * blockIdx.x + 1, mb, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        last = atomicAdd(state, 1) == (int)gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    __threadfence();
+    ma = t < (int)gridDim.x ? __hip_atomic_load(part + 2 * t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    mb = t < (int)gridDim.x ? __hip_atomic_load(part + 2 * t + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+    reduce(ma, mb);
+    const bool one = (long long)ma * mb <= bound;
+    for (int i = t; i < words; i += kOneBinThreads)
+        ctl[i] = !one ? 0u : i == set.x || i == set.y || i == set.z ? (uint32_t)M : i == one_word ? 1u : 0u;
+    if (t == 0) {
+        atomicExch(state, 0);
+        __hip_atomic_store(host, one ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        __threadfence_system();
+        __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
+void launch_one_bin(const SpOperand &A, const SpOperand &B, long long bound, int *part, int *state, int32_t *list,
+                    void *ctl, int words, int3 set, int one_word, unsigned *host, unsigned long long *flag,
+                    unsigned long long seq, hipStream_t st)
+{
+    const int64_t rows = std::max(A.M, B.M);
+    const unsigned g = (unsigned)std::min<int64_t>(kOneBinBlocks, (rows + kOneBinThreads - 1) / kOneBinThreads);
+    auto *w = static_cast<uint32_t *>(ctl);
+    if (A.rp32 && B.rp32)
+        hipLaunchKernelGGL((k_one_bin<int32_t, int32_t>), dim3(std::max(g, 1u)), dim3(kOneBinThreads), 0, st, A.rp32,
+                           A.M, B.rp32, B.M, bound, part, state, list, w, words, set, one_word, host, flag, seq);
+    else
+        hipLaunchKernelGGL((k_one_bin<int64_t, int64_t>), dim3(std::max(g, 1u)), dim3(kOneBinThreads), 0, st, A.rp,
+                           A.M, B.rp, B.M, bound, part, state, list, w, words, set, one_word, host, flag, seq);
+}
+
 // Upper bounds ub(r) = sum of nnz(B_k) over the entries k of row r of A, one
 // wavefront per row (four entries per lane in flight): for operators whose
 // rows run to hundreds of entries, where one thread per row would walk its
@@ -3327,6 +3421,137 @@ void launch_extract(const int64_t *rp, const int32_t *col, const double *val, in
                     int64_t *orp, int32_t *orp32, int32_t *ocol, double *oval, hipStream_t st)
 {
     hipLaunchKernelGGL(k_extract, dim3(256), dim3(256), 0, st, rp, col, val, r0, M, coloff, orp, orp32, ocol, oval);
+}
+
+// The end of a scan of row lengths and the gather behind it in one launch, for
+// plans whose rows sit in one bin's slots in row order (slot r: row r).  A
+// workgroup takes 512 / L rows: their offsets are the sums of the lengths
+// before them (tile_sums null: of the lengths themselves, at most
+// kScanGatherRows; else of the tile sums of k_scan_tiles, with the tile-local
+// offsets in `out`), and it then moves the rows.  Workgroup 0 stores the total
+// and, with xdst, copies xwords words of the control block to the host.
+// Rows whose slot is marked -1 have length 0 and are left to the caller.
+// With k_one_bin a small product is 3 launches instead of 8: 5-point 64^2 57 ->
+// 46 us, 7-point 61x47x53 (19,000 rows, with k_scan_tiles) 90 -> 84; 128^3
+// (262,144 rows) 595 us joint and 598 apart.
+constexpr int kScanGatherRows = 4096;
+template <int L>
+__global__ void __launch_bounds__(256) k_scan_gather(const int32_t *__restrict__ len, int64_t n,
+                                                     const long long *__restrict__ tile_sums, int ntiles,
+                                                     int64_t *__restrict__ out, int32_t *__restrict__ out32,
+                                                     int64_t *__restrict__ total_out,
+                                                     const int32_t *__restrict__ slotn, int cap,
+                                                     const int32_t *__restrict__ scol,
+                                                     const double *__restrict__ sval, int32_t *__restrict__ ccol,
+                                                     double *__restrict__ cval, int64_t out_cap,
+                                                     int *__restrict__ err, const uint32_t *xsrc, uint32_t *xdst,
+                                                     int xwords)
+{
+    constexpr int RPB = 512 / L;  // two rows per group of L lanes
+    static_assert(RPB <= 64 && kScanTile % RPB == 0, "a wavefront scans the rows, which lie in one tile");
+    __shared__ long long sp[256 / 64], sq[256 / 64];
+    __shared__ int64_t off[RPB];
+    const int t = threadIdx.x;
+    const int64_t r0 = (int64_t)blockIdx.x * RPB;
+    long long pre = 0, tot = 0;
+    if (tile_sums) {
+        const int tile = (int)(r0 / kScanTile);
+        for (int j = t; j < ntiles; j += 256) {
+            const long long v = tile_sums[j];
+            tot += v;
+            pre += j < tile ? v : 0;
+        }
+    } else {
+        for (int64_t j = t; j < n; j += 256) {
+            const int v = len[j];
+            tot += v;
+            pre += j < r0 ? v : 0;
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        pre += __shfl_xor(pre, o);
+        tot += __shfl_xor(tot, o);
+    }
+    if (lane() == 0) {
+        sp[t / 64] = pre;
+        sq[t / 64] = tot;
+    }
+    __syncthreads();
+    pre = sp[0] + sp[1] + sp[2] + sp[3];
+    tot = sq[0] + sq[1] + sq[2] + sq[3];
+    if (t < 64) {
+        const int64_t r = r0 + t;
+        const bool mine = t < RPB && r < n;
+        long long v = 0;
+        if (tile_sums) {
+            v = mine ? out[r] : 0;
+        } else {
+            const int own = mine ? len[r] : 0;
+            int inc = own;
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(inc, o);
+                if (t >= o) inc += y;
+            }
+            v = inc - own;
+        }
+        v += pre;
+        if (t < RPB) off[t] = v;
+        if (mine) {
+            out[r] = v;
+            if (out32 && tot < 2147483647LL) out32[r] = (int32_t)v;
+        }
+        if (t < RPB && r == n) {
+            out[n] = tot;
+            if (out32 && tot < 2147483647LL) out32[n] = (int32_t)tot;
+        }
+        if (blockIdx.x == 0 && t == 0) {
+            *total_out = tot;
+            __threadfence();  // exported below
+        }
+    }
+    __syncthreads();
+    if (xdst && blockIdx.x == 0)
+        for (int i = t; i < xwords; i += 256) xdst[i] = xsrc[i];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int k = u * (256 / L) + t / L;
+        const int64_t r = r0 + k;
+        const int m = r < n ? slotn[r] : 0;
+        if (m <= 0) continue;
+        const int64_t src = r * cap, dst = off[k];
+        if (dst + m > out_cap) {  // output smaller than this product needs
+            if (t % L == 0) atomicOr(err, kErrOverflow);
+            continue;
+        }
+        for (int j = t % L; j < m; j += L) {
+            ccol[dst + j] = scol[src + j];
+            cval[dst + j] = sval[src + j];
+        }
+    }
+}
+
+// the tile sums fit one step of a workgroup's lanes
+bool scan_gather_fits(int64_t n) { return n > 0 && n <= 256 * (int64_t)kScanTile; }
+
+void launch_scan_gather(const int32_t *len, int64_t n, int64_t *out, int32_t *out32, long long *tile_sums,
+                        int64_t *total, const int32_t *slotn, int cap, const int32_t *scol, const double *sval,
+                        int32_t *ccol, double *cval, int64_t out_cap, int *err, const void *xsrc, void *xdst,
+                        int xwords, hipStream_t st)
+{
+    const int ntiles = (int)((n + kScanTile - 1) / kScanTile);
+    const long long *sums = nullptr;
+    if (n > kScanGatherRows) {
+        hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)ntiles), dim3(kScanThreads), 0, st, len, n, out, tile_sums);
+        sums = tile_sums;
+    }
+    const auto *xs = static_cast<const uint32_t *>(xsrc);
+    auto *xd = static_cast<uint32_t *>(xdst);
+    if (cap <= 128)
+        hipLaunchKernelGGL(k_scan_gather<16>, dim3(blocks_for(n + 1, 512 / 16)), dim3(256), 0, st, len, n, sums,
+                           ntiles, out, out32, total, slotn, cap, scol, sval, ccol, cval, out_cap, err, xs, xd, xwords);
+    else
+        hipLaunchKernelGGL(k_scan_gather<32>, dim3(blocks_for(n + 1, 512 / 32)), dim3(256), 0, st, len, n, sums,
+                           ntiles, out, out32, total, slotn, cap, scol, sval, ccol, cval, out_cap, err, xs, xd, xwords);
 }
 
 void launch_scan(const int32_t *in, int64_t n, int64_t *out, int32_t *out32, long long *tile_sums,

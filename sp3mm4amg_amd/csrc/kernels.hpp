@@ -66,6 +66,11 @@ void launch_ub_bin(const SpOperand &A, const SpOperand &B, int64_t *ub, int32_t 
                    const OneBin *one = nullptr, bool wave_ub = false);
 // wave_ub: the bounds are measured a wavefront per row of A first (rows of
 // A averaging kWaveUbRow entries or more), then binned
+// One-bin mode decided by one launch (see k_one_bin): host[0] = 1 when every row
+// fits `bound`, then *flag = seq.  state: a word that is zero between launches.
+void launch_one_bin(const SpOperand &A, const SpOperand &B, long long bound, int *part, int *state, int32_t *list,
+                    void *ctl, int words, int3 set, int one_word, unsigned *host, unsigned long long *flag,
+                    unsigned long long seq, hipStream_t st);
 void launch_ub_colparts(const int64_t *arp, const int32_t *acol, int64_t M, const int64_t *boff, int G,
                         int64_t *out, unsigned long long *total, hipStream_t st);
 void launch_rebin(const int32_t *m1, const int32_t *m2, int64_t M, int32_t *lists, int *counts,
@@ -241,6 +246,13 @@ void launch_extract(const int64_t *rp, const int32_t *col, const double *val, in
                     int64_t *orp, int32_t *orp32, int32_t *ocol, double *oval, hipStream_t st);
 
 int64_t scan_tiles(int64_t n);
+// launch_scan and the gather of one bin's slots (slot r: row r) in one or two
+// launches, for at most 524,288 rows (scan_gather_fits)
+bool scan_gather_fits(int64_t n);
+void launch_scan_gather(const int32_t *len, int64_t n, int64_t *out, int32_t *out32, long long *tile_sums,
+                        int64_t *total, const int32_t *slotn, int cap, const int32_t *scol, const double *sval,
+                        int32_t *ccol, double *cval, int64_t out_cap, int *err, const void *xsrc, void *xdst,
+                        int xwords, hipStream_t st);
 void launch_scan(const int32_t *in, int64_t n, int64_t *out, int32_t *out32, long long *tile_sums,
                  int64_t *total, hipStream_t st);
 
