@@ -2669,8 +2669,10 @@ __global__ void __launch_bounds__(kWin) k_window_direct(SpOperand R, SpOperand A
     const int S = 1 << slog1;
     // list entries i index the per-row slots: at most cap_rows of them
     const int n = clamp_count(count, cap_rows, err);
-    const RowWalk walk = row_walk<1>(n, 0, nxcd);
-    for (int i = walk.i; i < walk.end; i += walk.stride) {
+    // one row per workgroup and round; of the rows of a round, neighbours on one
+    // XCD (workgroup b runs on XCD b % nxcd)
+    const int first = (int)blockIdx.x % nxcd * ((int)gridDim.x / nxcd) + (int)blockIdx.x / nxcd;
+    for (int i = first; i < n; i += gridDim.x) {
         const int r = rows[i];
         const int64_t e0 = R.rp[r], e1 = R.rp[r + 1];
         // window of the R*A row
@@ -2932,9 +2934,11 @@ void launch_window_direct(bool num, int blocks, size_t lds, const SpOperand &R, 
     // workgroup (64 lanes each, 16 in flight, made the 1728-row level of a
     // 96^3 hierarchy 6% slower)
     if (slog1 > 4) slog1 = 4;
-    // neighbouring rows on one XCD's L2 (1728 rows of a 96^3 hierarchy: 400 -> 124
-    // MB fetched per product); a grid that is no multiple of the XCDs has a row
-    // per workgroup and needs every one of them
+    // neighbouring rows of a round on one XCD's L2 (1728 rows of a 96^3 hierarchy:
+    // 498 instead of 527 us); a grid that is no multiple of the XCDs has a row
+    // per workgroup and needs every one of them.  Not an eighth of the list per
+    // XCD: the long rows of several levels in one list are uneven (batch of a
+    // 4-level 96^3 hierarchy and 64 small products: 1.76 ms by eighths, 1.48)
     const int nxcd = blocks % kXcds == 0 ? kXcds : 1;
 #define SP3MM_WIN_ARGS R, A, P, rows, count, cap, slog1, nxcd, spill, nspill, rownnz, crp, ccol, cval, rowsum, out_cap, \
                        err, slotn, scol, sval, cap_rows
