@@ -145,9 +145,10 @@ __global__ void __launch_bounds__(256) k_row_maxlen(const IA *__restrict__ arp, 
 // kernel queued behind this one at once), and tells the host.  The list of the
 // bin is every row in order.  Replaces four launches of 3 to 5 us each, two
 // thirds of what a small product runs before its main kernel.
-// 64 workgroups: one addition each to the ticket, at 15 ns (state[0]; zero
-// before and after), and 1024 lanes with four rows in flight.
-constexpr int kOneBinBlocks = 64, kOneBinThreads = 1024;
+// Workgroups of 1024 lanes, four rows in flight each: 64, and from 524,288 rows
+// on one per 8192, up to 256 (each adds to the ticket, state[0], at 15 ns; it
+// is zero before and after).  2,097,152 rows: 23 us by 64, 17 by 256.
+constexpr int kOneBinBlocks = 256, kOneBinThreads = 1024;
 static_assert(kOneBinBlocks <= kMaxLenBlocks && kOneBinBlocks <= kOneBinThreads, "a partial per lane");
 template <typename IA, typename IB>
 __global__ void __launch_bounds__(kOneBinThreads) k_one_bin(const IA *__restrict__ arp, int64_t M,
@@ -222,7 +223,8 @@ void launch_one_bin(const SpOperand &A, const SpOperand &B, long long bound, int
                     unsigned long long seq, hipStream_t st)
 {
     const int64_t rows = std::max(A.M, B.M);
-    const unsigned g = (unsigned)std::min<int64_t>(kOneBinBlocks, (rows + kOneBinThreads - 1) / kOneBinThreads);
+    const unsigned g = (unsigned)std::min<int64_t>(std::min<int64_t>(kOneBinBlocks, std::max<int64_t>(64, rows / 8192)),
+                                                   (rows + kOneBinThreads - 1) / kOneBinThreads);
     auto *w = static_cast<uint32_t *>(ctl);
     if (A.rp32 && B.rp32)
         hipLaunchKernelGGL((k_one_bin<int32_t, int32_t>), dim3(std::max(g, 1u)), dim3(kOneBinThreads), 0, st, A.rp32,

@@ -42,7 +42,7 @@ def test_one_bin(m, la, lp, kind):
         assert np.all(np.abs(got.vals - want.vals) <= bound)
 
 
-@pytest.mark.parametrize("m", [524288, 524289])
+@pytest.mark.parametrize("m", [524288, 524289, 700001])
 def test_rows_around_the_joint_limit(m):
     """R selects one row of A per row, so the product is A*P's rows repeated."""
     rng = np.random.default_rng(3)
