@@ -7,6 +7,7 @@
 #include <cstdlib>
 
 #include "device_common.hpp"
+#include "jacobi_plan.hpp"
 #include "kernels.hpp"
 
 namespace sp3mm {
@@ -762,13 +763,14 @@ static size_t jacobi_small_lds(int64_t M, int64_t nnz) { return (size_t)nnz * 12
 // produces (hardware quiets NaN results), and the next sweep polls every entry
 // until it is there: the data is its own flag, so a sweep costs one store
 // reaching one load (agent scope) and no barrier across workgroups.  The last
-// sweep writes x.  At most 256 workgroups of 512 lanes and 34 KB of LDS: all
+// sweep writes x, behind the polls of the sweep before it, which wait for every
+// workgroup's read of x: a launch takes two sweeps at least (jacobi_chunk).  At most 256 workgroups of 512 lanes and 34 KB of LDS: all
 // fit the 256 CUs at once, and a poll that does not see its entry within
 // kGridSpins loads gives up with kErrSpin, so every wave ends.  Rows are
 // summed in k_jacobi's order (equal results).  50 sweeps in a V-cycle's graph,
 // 512 rows: 330 -> 163 us; called alone 267 -> 183, 1,000 rows 255 -> 223.
 // Two or four rows per group (fewer workgroups polling): 192 to 525 us.
-constexpr int kGridRows = 2048, kGridThreads = 512, kGridRegs = 8, kGridSweeps = 64;
+constexpr int kGridRows = 2048, kGridThreads = 512, kGridRegs = 8;
 constexpr unsigned long long kGridEmpty = 0x7FF7A5A57FF7A5A5ull;
 constexpr int kGridSpins = 1 << 21;
 
@@ -915,9 +917,9 @@ bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val
     if (M <= 0 || M > kGridRows || sweeps < kGridMin || !buf) return false;
     const int L = lanes_for(M, nnz);
     auto *w = static_cast<unsigned long long *>(buf);
-    for (int k = 0; k < sweeps; k += kGridSweeps) {
-        const int n = std::min(kGridSweeps, sweeps - k);
-        if (n > 1) hipLaunchKernelGGL(k_grid_empty, dim3(grid1((n - 1) * M)), dim3(256), 0, st, w, (int64_t)(n - 1) * M);
+    for (int k = 0, n; k < sweeps; k += n) {
+        n = jacobi_chunk(sweeps - k);
+        hipLaunchKernelGGL(k_grid_empty, dim3(grid1((n - 1) * M)), dim3(256), 0, st, w, (int64_t)(n - 1) * M);
         const unsigned g = grid1(M, kGridThreads / L);
         SP3MM_BY_LANES(k_jacobi_grid, dim3(g), dim3(kGridThreads), 0, st, rp, col, val, (int)M, b, x, w, omega, n,
                        from_zero && k == 0, err)
