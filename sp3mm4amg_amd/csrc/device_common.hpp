@@ -22,7 +22,6 @@ enum : int {
     kErrHashFull = 1,     // an LDS hash table ran out of slots (sizing bug)
     kErrOverflow = 2,     // an output row did not fit the space reserved for it
     kErrBadInput = 4,     // input validation failed
-    kErrSpin = 8,         // a bounded wait gave up
     kErrLongRow = 16,     // a row is longer than the kernel takes (the caller has another path)
 };
 

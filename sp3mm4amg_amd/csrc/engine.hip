@@ -139,6 +139,19 @@ static void tuning_from_env(Tuning &t)
 
 static bool same_tuning(const Tuning &a, const Tuning &b);
 
+// CUs that the current stream's kernels may run on: those of its CU mask
+static int usable_cus(const Context *c)
+{
+    uint32_t mask[32] = {};
+    if (hipExtStreamGetCUMask(c->stream, 32, mask) != hipSuccess) {
+        (void)hipGetLastError();
+        return c->num_cu;
+    }
+    int n = 0;
+    for (uint32_t m : mask) n += __builtin_popcount(m);
+    return n > 0 ? std::min(n, c->num_cu) : c->num_cu;
+}
+
 int init_device(int dev)
 {
     std::lock_guard<std::mutex> lk(g_ctx_mu);
@@ -173,6 +186,7 @@ int init_device(int dev)
     c->adapt = same_tuning(c->tune, Tuning{});
     SP3MM_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
     c->stream = c->own_stream;
+    c->stream_cus = usable_cus(c);
     SP3MM_HIP(hipHostMalloc((void **)&c->host_small, 4096, hipHostMallocDefault));
     // a coherent block the host polls for counters exported mid-stream (null:
     // the plans read their counters back with a stream synchronisation)
@@ -2426,6 +2440,7 @@ int set_stream(hipStream_t s)
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     SP3MM_HIP(hipStreamSynchronize(c->stream));
     c->stream = s ? s : c->own_stream;
+    c->stream_cus = usable_cus(c);
     return 0;
 }
 
@@ -2477,8 +2492,7 @@ int consumer_wait(Context *c, double *dot_out)
         ConsState *d = static_cast<ConsState *>(c->cons);
         SP3MM_HIP(hipMemsetAsync(&d->err, 0, sizeof(int), c->stream));
         SP3MM_HIP(hipStreamSynchronize(c->stream));
-        if (h.err & kErrSpin) set_error("jacobi: a sweep waited in vain for another workgroup's rows");
-        else set_error("jacobi: zero diagonal entry (sweep launched before this call)");
+        set_error("jacobi: zero diagonal entry (sweep launched before this call)");
         return -1;
     }
     return 0;
@@ -2559,7 +2573,7 @@ void queue_jacobi(const sp3mm_dmat &A, const double *b, double *x, double *work,
     const double *val = static_cast<const double *>(A.val);
     const bool small = sweeps > 1 && jacobi_small_fits(A.M, A.nnz, ctx()->lds_device);
     if (!small && launch_jacobi_grid(A.rp, A.col, val, A.M, A.nnz, b, x, jacobi_buffers(ctx()), omega, sweeps,
-                                     from_zero, err, s))
+                                     from_zero, err, ctx()->stream_cus, s))
         return;
     if (from_zero && (small || sweeps == 0)) launch_axpby(A.M, 0.0, nullptr, 0.0, x, s);
     if (small) {

@@ -56,6 +56,7 @@ struct Context {
     hipStream_t stream = nullptr;      // the stream every call is queued on
     hipStream_t own_stream = nullptr;  // the library's own (non-blocking) stream
     int num_cu = 0;
+    int stream_cus = 0;                // CUs that `stream` may use (num_cu unless its CU mask holds fewer)
     size_t max_lds = 65536;
     size_t lds_device = 65536;
     Pool pool;

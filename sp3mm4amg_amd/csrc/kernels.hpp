@@ -305,7 +305,7 @@ void launch_spmv(const int64_t *rp, const int32_t *col, const double *val, int64
 // otherwise)
 bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
                         const double *b, double *x, void *buf, double omega, int sweeps, bool from_zero, int *err,
-                        hipStream_t st);
+                        int cus, hipStream_t st);
 size_t jacobi_grid_bytes();  // of `buf`
 bool jacobi_small_fits(int64_t M, int64_t nnz, size_t max_lds);
 // one sweep from x = 0 into xo

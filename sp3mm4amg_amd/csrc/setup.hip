@@ -4,6 +4,7 @@
 // The reference receives P and R from its caller; these kernels let a whole
 // hierarchy be built level after level without leaving HBM.
 #include <algorithm>
+#include <atomic>
 #include <cstdlib>
 
 #include "device_common.hpp"
@@ -764,15 +765,23 @@ static size_t jacobi_small_lds(int64_t M, int64_t nnz) { return (size_t)nnz * 12
 // until it is there: the data is its own flag, so a sweep costs one store
 // reaching one load (agent scope) and no barrier across workgroups.  The last
 // sweep writes x, behind the polls of the sweep before it, which wait for every
-// workgroup's read of x: a launch takes two sweeps at least (jacobi_chunk).  At most 256 workgroups of 512 lanes and 34 KB of LDS: all
-// fit the 256 CUs at once, and a poll that does not see its entry within
-// kGridSpins loads gives up with kErrSpin, so every wave ends.  Rows are
-// summed in k_jacobi's order (equal results).  50 sweeps in a V-cycle's graph,
+// workgroup's read of x: a launch takes two sweeps at least (jacobi_chunk).
+// The sweeps need their workgroups (at most 256 of 512 lanes and 34 KB of LDS)
+// on the chip together; the launcher takes this form only where the stream's
+// CUs hold them all (jacobi_grid_resident).  Other work can still keep some
+// from starting, so a poll that does not see its entry within kGridSpins loads
+// (some 50 ms) gives up, every other one then does, too, and k_jacobi_redo
+// behind it runs all the sweeps in one workgroup from the copy of x that
+// k_grid_empty took (otherwise it ends at once; counting the workgroups that
+// end, to redo the sweeps in the last one, cost 7 to 30 us a launch in fences).
+// Rows are summed in k_jacobi's order either way (equal results).  50 sweeps in a V-cycle's graph,
 // 512 rows: 330 -> 163 us; called alone 267 -> 183, 1,000 rows 255 -> 223.
 // Two or four rows per group (fewer workgroups polling): 192 to 525 us.
-constexpr int kGridRows = 2048, kGridThreads = 512, kGridRegs = 8;
+constexpr int kGridRegs = 8;
 constexpr unsigned long long kGridEmpty = 0x7FF7A5A57FF7A5A5ull;
-constexpr int kGridSpins = 1 << 21;
+constexpr int kGridSpins = 1 << 16;
+// behind the sweeps' buffers: x as it was, and the word of a poll that gave up
+constexpr size_t kGridCopy = (size_t)(kGridSweeps - 1) * kGridRows, kGridWords = kGridCopy + kGridRows + 1;
 
 template <int L>
 __global__ void __launch_bounds__(kGridThreads) k_jacobi_grid(const int64_t *__restrict__ rp,
@@ -780,10 +789,11 @@ __global__ void __launch_bounds__(kGridThreads) k_jacobi_grid(const int64_t *__r
                                                               const double *__restrict__ val, int M,
                                                               const double *__restrict__ b, double *x,
                                                               unsigned long long *buf, double omega, int sweeps,
-                                                              bool from_zero, int *__restrict__ err)
+                                                              bool from_zero, int spins, int *__restrict__ err)
 {
     __shared__ double xs[2][kGridRows];
     __shared__ int dead;
+    int *gave_up = reinterpret_cast<int *>(buf + kGridCopy + kGridRows);
     const int t = threadIdx.x, sub = t & (L - 1);
     const int r = blockIdx.x * (kGridThreads / L) + t / L;
     const bool act = r < M;
@@ -830,9 +840,10 @@ __global__ void __launch_bounds__(kGridThreads) k_jacobi_grid(const int64_t *__r
         double *xo = xs[(k + 1) & 1];
         for (int i = t; i < M; i += kGridThreads) {
             unsigned long long w = kGridEmpty;
-            for (int n = 0; n < kGridSpins; n++) {
+            for (int n = 0; n < spins; n++) {
                 w = __hip_atomic_load(buf + (int64_t)k * M + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (w != kGridEmpty) break;
+                if ((n & 1023) == 1023 && __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) break;
                 __builtin_amdgcn_s_sleep(1);
             }
             if (w == kGridEmpty) dead = 1;
@@ -840,19 +851,79 @@ __global__ void __launch_bounds__(kGridThreads) k_jacobi_grid(const int64_t *__r
         }
         __syncthreads();
         if (dead) {  // uniform: written before the barrier
-            if (t == 0) atomicOr(err, kErrSpin);
+            if (t == 0) __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return;
         }
     }
 }
 
-__global__ void k_grid_empty(unsigned long long *p, int64_t n)
+// the sweeps of a k_jacobi_grid that gave up, in one workgroup
+template <int L>
+__global__ void __launch_bounds__(1024) k_jacobi_redo(const int64_t *__restrict__ rp, const int32_t *__restrict__ col,
+                                                       const double *__restrict__ val, int M,
+                                                       const double *__restrict__ b, double *__restrict__ x,
+                                                       const unsigned long long *__restrict__ buf, double omega,
+                                                       int sweeps, bool from_zero)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = kGridEmpty;
+    __shared__ double xs[2][kGridRows];
+    if (*reinterpret_cast<const int *>(buf + kGridCopy + kGridRows) == 0) return;
+    const int t = threadIdx.x, sub = t & (L - 1);
+    for (int i = t; i < M; i += 1024)
+        xs[0][i] = from_zero ? 0.0 : __longlong_as_double((long long)buf[kGridCopy + i]);
+    __syncthreads();
+    for (int k = 0; k < sweeps; k++) {
+        const double *xi = xs[k & 1];
+        double *xo = xs[(k + 1) & 1];
+        for (int q = t / L; q < M; q += 1024 / L) {
+            double s = 0.0, dq = 0.0;
+            for (int64_t e = rp[q] + sub; e < rp[q + 1]; e += L) {
+                const int ce = col[e];
+                s += val[e] * xi[ce];
+                if (ce == q) dq = val[e];
+            }
+            for (int o = L / 2; o > 0; o >>= 1) {
+                s += __shfl_xor(s, o);
+                dq += __shfl_xor(dq, o);
+            }
+            if (sub == 0) xo[q] = dq == 0.0 ? xi[q] : xi[q] + omega * (b[q] - s) / dq;
+        }
+        __syncthreads();
+    }
+    for (int i = t; i < M; i += 1024) x[i] = xs[sweeps & 1][i];
 }
 
-size_t jacobi_grid_bytes() { return (size_t)(kGridSweeps - 1) * kGridRows * 8; }
+__global__ void k_grid_empty(unsigned long long *buf, int64_t n, const double *__restrict__ x, int M)
+{
+    const int64_t i0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = i0; i < n; i += step) buf[i] = kGridEmpty;
+    for (int64_t i = i0; i < M; i += step) buf[kGridCopy + i] = (unsigned long long)__double_as_longlong(x[i]);
+    if (i0 == 0) buf[kGridCopy + kGridRows] = 0;
+}
+
+size_t jacobi_grid_bytes() { return kGridWords * 8; }
+
+// workgroups of k_jacobi_grid<L> that one CU holds, 0 if unknown
+static int grid_per_cu(int L)
+{
+    static std::atomic<int> known[7];  // by log2 of L: the count, plus one
+    std::atomic<int> &k = known[ilog2((unsigned)L)];
+    int n = k.load(std::memory_order_relaxed) - 1;
+    if (n >= 0) return n;
+    auto occ = [&](auto fn) { return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, kGridThreads, 0); };
+    const hipError_t e = L == 1    ? occ(k_jacobi_grid<1>)
+                         : L == 2  ? occ(k_jacobi_grid<2>)
+                         : L == 4  ? occ(k_jacobi_grid<4>)
+                         : L == 8  ? occ(k_jacobi_grid<8>)
+                         : L == 16 ? occ(k_jacobi_grid<16>)
+                         : L == 32 ? occ(k_jacobi_grid<32>)
+                                   : occ(k_jacobi_grid<64>);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    k.store(n + 1, std::memory_order_relaxed);
+    return n;
+}
 
 // Lanes per row: the smallest power of two (at most 64) not below the mean
 // row length divided by SP3MM_SPMV_ROW_DIV (default 4: about four entries
@@ -907,22 +978,29 @@ bool jacobi_small_fits(int64_t M, int64_t nnz, size_t max_lds)
 }
 
 // Launches nothing and returns false when a launch per sweep is as good: fewer
-// than kGridMin sweeps (clearing the buffers is a launch of its own), or rows
-// beyond what 256 workgroups hold.
+// than kGridMin sweeps (clearing the buffers is a launch of its own), or more
+// workgroups than the `cus` CUs at hand hold together.  SP3MM_GRID_SPINS: loads
+// after which a poll gives up.
 bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
                         const double *b, double *x, void *buf, double omega, int sweeps, bool from_zero, int *err,
-                        hipStream_t st)
+                        int cus, hipStream_t st)
 {
     constexpr int kGridMin = 4;
-    if (M <= 0 || M > kGridRows || sweeps < kGridMin || !buf) return false;
+    if (M <= 0 || sweeps < kGridMin || !buf) return false;
     const int L = lanes_for(M, nnz);
+    if (M > kGridRows || !jacobi_grid_resident((int)M, L, grid_per_cu(L), cus)) return false;
+    const char *env = getenv("SP3MM_GRID_SPINS");
+    const int spins = env ? std::max(0, atoi(env)) : kGridSpins;
     auto *w = static_cast<unsigned long long *>(buf);
     for (int k = 0, n; k < sweeps; k += n) {
         n = jacobi_chunk(sweeps - k);
-        hipLaunchKernelGGL(k_grid_empty, dim3(grid1((n - 1) * M)), dim3(256), 0, st, w, (int64_t)(n - 1) * M);
+        hipLaunchKernelGGL(k_grid_empty, dim3(grid1((n - 1) * M)), dim3(256), 0, st, w, (int64_t)(n - 1) * M, x,
+                           from_zero && k == 0 ? 0 : (int)M);
         const unsigned g = grid1(M, kGridThreads / L);
         SP3MM_BY_LANES(k_jacobi_grid, dim3(g), dim3(kGridThreads), 0, st, rp, col, val, (int)M, b, x, w, omega, n,
-                       from_zero && k == 0, err)
+                       from_zero && k == 0, spins, err)
+        SP3MM_BY_LANES(k_jacobi_redo, dim3(1), dim3(1024), 0, st, rp, col, val, (int)M, b, x, w, omega, n,
+                       from_zero && k == 0)
     }
     return true;
 }

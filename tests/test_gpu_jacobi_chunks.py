@@ -24,3 +24,24 @@ def test_sweeps_equal_single_sweeps(m, per_row, sweeps):
             L.jacobi(dA, db, dx, dw, 0.6, n)
         got.append(dx.numpy())
     assert np.array_equal(*got)
+
+
+@pytest.mark.parametrize("m,per_row,sweeps", [(2048, 520, 65), (513, 300, 4), (1200, 40, 50)])
+def test_sweeps_whose_polls_give_up(m, per_row, sweeps, monkeypatch):
+    # no loads allowed: every workgroup gives up at its first poll that is not
+    # answered at once, and the last one to end runs the sweeps alone
+    rng = np.random.default_rng(sweeps)
+    dA = L.DeviceCSR.upload(_dominant(m, np.full(m, per_row), m))
+    b, x = rng.standard_normal(m), rng.standard_normal(m)
+    db, dw = L.DeviceArray.from_numpy(b), L.DeviceArray(m)
+    got = []
+    for spins in ("0", None):
+        if spins:
+            monkeypatch.setenv("SP3MM_GRID_SPINS", spins)
+        else:
+            monkeypatch.delenv("SP3MM_GRID_SPINS")
+        dx = L.DeviceArray.from_numpy(x)
+        L.jacobi(dA, db, dx, dw, 0.6, sweeps)
+        L.sync()
+        got.append(dx.numpy())
+    assert np.array_equal(*got)

@@ -28,3 +28,13 @@ def test_no_launch_of_one_sweep(tmp_path):
     assert [r[0] for r in rows] == list(range(4, 401))
     for s, *chunks in rows:
         assert sum(chunks) == s and all(2 <= n <= 64 for n in chunks), (s, chunks)
+
+
+def test_launch_needs_all_its_workgroups_on_the_chip(tmp_path):
+    # 64 lanes per row: 8 rows per workgroup; 256 workgroups do not fit 32 CUs of 4
+    out = _run(tmp_path, "const int q[][4] = {{2048, 64, 4, 256}, {2048, 64, 4, 64}, {2048, 64, 4, 63}, {2048, 64, 4, 32},"
+                         "{513, 64, 1, 64}, {513, 64, 1, 65}, {2048, 1, 4, 1}, {2048, 64, 0, 256}};\n"
+                         "for (auto &v : q) std::printf(\"%d %d\\n\", jacobi_groups(v[0], v[1]),"
+                         " (int)jacobi_grid_resident(v[0], v[1], v[2], v[3]));")
+    got = [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+    assert got == [(256, 1), (256, 1), (256, 0), (256, 0), (65, 0), (65, 1), (4, 1), (256, 0)]
