@@ -451,13 +451,17 @@ int sp3mm_set_tuning(const sp3mm_tuning *t);
 /* Autotuner: times the direct product R*A*P (opts->precision as in sp3mm_rap)
  * under candidate schedules, `reps` products each, and installs the fastest
  * for later calls; *best receives it, *ms_best and *ms_default the median
- * device times of the chosen and of the starting schedule. */
+ * device times of the chosen and of the starting schedule.  While the defaults
+ * stand the start is timed as it runs, adapted to the operands, and a candidate
+ * has to be faster than that to be installed: if none is, the defaults (*best)
+ * go on to be adapted. */
 int sp3mm_autotune(const sp3mm_dmat *R, const sp3mm_dmat *A, const sp3mm_dmat *P,
                    const sp3mm_opts *opts, int32_t reps, sp3mm_tuning *best,
                    double *ms_best, double *ms_default);
 /* The same on a batch's packed product (with the batch's precision); the
  * schedule found is installed and the batch (and its graph) rebuilt under
- * it. */
+ * it.  While the defaults stand, *ms_best and *ms_default are times of the
+ * batch's runs. */
 int sp3mm_batch_autotune(sp3mm_batch *b, int32_t reps, sp3mm_tuning *best,
                          double *ms_best, double *ms_default);
 

@@ -2728,17 +2728,44 @@ static bool same_tuning(const Tuning &x, const Tuning &y)
 // first tries the hash multipliers ranked on the operands (score_hashes).
 // The descent runs from the installed schedule and again from two presets
 // (mesh operators; tables at an eighth of the bound); the fastest end point
-// wins.
+// wins.  All of that takes schedules as they stand; where the starting one is
+// adapted to the operands (Context::adapt), autotune() and batch_autotune()
+// compare the end point with that afterwards.
 // --------------------------------------------------------------------------
-int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int prec, double guard, int reps,
-             Tuning &best, double &ms_best, double &ms_default)
+
+// Median device time of `n` products under each of two settings, interleaved.
+struct Setting {
+    Tuning tune;
+    bool adapt;
+};
+static int time_settings(Context *c, const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int prec,
+                         double guard, int n, const Setting (&set)[2], double (&ms)[2])
 {
-    Context *c = ctx();
-    if (!c) return -1;
-    std::lock_guard<std::recursive_mutex> lk(c->mu);
-    reps = std::min(std::max(reps, 1), 50);
+    std::vector<double> v[2];
+    for (int k = 0; k < n; k++) {
+        for (int w = 0; w < 2; w++) {
+            c->tune = set[w].tune;
+            c->adapt = set[w].adapt;
+            sp3mm_dmat C{};
+            sp3mm_stats st{};
+            const int rc = rap_direct_fused(R, A, P, C, &st, prec, guard > 0 ? guard : 1e-2, nullptr, false);
+            dmat_release(C);
+            if (rc) return -1;
+            v[w].push_back(st.ms_total);
+        }
+    }
+    for (int w = 0; w < 2; w++) {
+        std::sort(v[w].begin(), v[w].end());
+        ms[w] = v[w][v[w].size() / 2];
+    }
+    return 0;
+}
+
+// leaves the end point in c->tune (the start after an error), c->adapt as it was
+static int tune_schedule(Context *c, const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int prec,
+                         double guard, int reps, Tuning &best, double &ms_best, double &ms_default)
+{
     const Tuning saved = c->tune;
-    // candidates are timed as they stand; a schedule the tuner installs stays
     struct Fixed {
         Context *c;
         bool was;
@@ -2774,22 +2801,10 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
     // schedule, interleaved (2*reps runs each, medians): one noisy median of a
     // few runs does not decide the step
     auto confirm = [&](const Tuning &t, const Tuning &u, double &ms_t, double &ms_u) -> int {
-        std::vector<double> vt, vu;
-        for (int k = 0; k < 2 * reps + 1; k++) {
-            for (int w = 0; w < 2; w++) {
-                c->tune = w ? u : t;
-                sp3mm_dmat C{};
-                sp3mm_stats st{};
-                const int rc = rap_direct_fused(R, A, P, C, &st, prec, guard > 0 ? guard : 1e-2, nullptr, false);
-                dmat_release(C);
-                if (rc) return -1;
-                (w ? vu : vt).push_back(st.ms_total);
-            }
-        }
-        std::sort(vt.begin(), vt.end());
-        std::sort(vu.begin(), vu.end());
-        ms_t = vt[vt.size() / 2];
-        ms_u = vu[vu.size() / 2];
+        double ms[2];
+        if (time_settings(c, R, A, P, prec, guard, 2 * reps + 1, {{t, false}, {u, false}}, ms)) return -1;
+        ms_t = ms[0];
+        ms_u = ms[1];
         return 0;
     };
     Tuning cur = saved;
@@ -3005,7 +3020,7 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
         }
     }
     // the choice against the start once more, interleaved: a start that is not
-    // slower stays (the two were timed minutes of products apart)
+    // slower stays (the two were timed hundreds of products apart)
     if (!same_tuning(endb, saved)) {
         double ms_end = 0;
         if (confirm(saved, endb, ms_default, ms_end)) {
@@ -3022,10 +3037,35 @@ int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int 
         endb_ms = ms_default;
     }
     c->tune = endb;
-    fixed.was = false;
     best = endb;
     ms_best = endb_ms;
     return 0;
+}
+
+// A schedule the tuner installs is used as it is (adapt off).  Where the start
+// adapts to the operands, the end point replaces it only if it is at least 1%
+// faster than the adapted products: sampled tables and the unmerged forwarding
+// are no schedule the descent could reach (10,000-row lognormal operator:
+// 0.85 ms adapted, 1.36 for the best schedule).
+int autotune(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, int prec, double guard, int reps,
+             Tuning &best, double &ms_best, double &ms_default)
+{
+    Context *c = ctx();
+    if (!c) return -1;
+    std::lock_guard<std::recursive_mutex> lk(c->mu);
+    reps = std::min(std::max(reps, 1), 50);
+    const Setting start{c->tune, c->adapt};
+    if (tune_schedule(c, R, A, P, prec, guard, reps, best, ms_best, ms_default)) return -1;
+    if (!start.adapt) return 0;
+    double ms[2];
+    const int rc = time_settings(c, R, A, P, prec, guard, 2 * reps + 1, {start, {best, false}}, ms);
+    const bool faster = rc == 0 && ms[1] < 0.99 * ms[0] && !(prec == SP3MM_PREC_MIXED && same_tuning(best, start.tune));
+    if (!faster) best = start.tune;
+    c->tune = best;
+    c->adapt = !faster;
+    ms_default = ms[0];
+    ms_best = faster ? ms[1] : ms[0];
+    return rc;
 }
 
 // --------------------------------------------------------------------------
@@ -3240,17 +3280,45 @@ int batch_autotune(void *h, int reps, Tuning &best, double &ms_best, double &ms_
     if (!c || !h) return -1;
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     Batch *b = static_cast<Batch *>(h);
-    if (autotune(b->Rb, b->Ab, b->Pb, b->prec, b->guard, reps, best, ms_best, ms_default)) return -1;
-    // rebuild the plan (and the graph, if there was one) for the schedule found
+    reps = std::min(std::max(reps, 1), 50);
+    // rebuilds the plan (and the graph, if there was one) under the context's
+    // schedule; with `ms`, also the median device time of its runs
     const bool graph = b->exec != nullptr;
-    SP3MM_HIP(hipStreamSynchronize(c->stream));
-    if (b->exec) (void)hipGraphExecDestroy(b->exec);
-    if (b->graph) (void)hipGraphDestroy(b->graph);
-    b->exec = nullptr;
-    b->graph = nullptr;
-    b->plan.release_all();
-    b->plan = FusedPlan();
-    return batch_build(c, b, graph);
+    auto rebuild = [&](double *ms) -> int {
+        SP3MM_HIP(hipStreamSynchronize(c->stream));
+        if (b->exec) (void)hipGraphExecDestroy(b->exec);
+        if (b->graph) (void)hipGraphDestroy(b->graph);
+        b->exec = nullptr;
+        b->graph = nullptr;
+        b->plan.release_all();
+        b->plan = FusedPlan();
+        if (batch_build(c, b, graph)) return -1;
+        std::vector<double> v;
+        for (int k = 0; ms && k < 2 * reps + 1; k++) {
+            double t = 0;
+            if (batch_run(b, b->exec != nullptr, &t)) return -1;
+            v.push_back(t);
+        }
+        std::sort(v.begin(), v.end());
+        if (ms) *ms = v[v.size() / 2];
+        return 0;
+    };
+    // as in autotune(), the start's and the end point's runs compared: the runs
+    // do not sample their rows again, which single products do
+    const Setting start{c->tune, c->adapt};
+    double ms_start = 0, ms_end = 0;
+    if (start.adapt && rebuild(&ms_start)) return -1;
+    if (tune_schedule(c, b->Rb, b->Ab, b->Pb, b->prec, b->guard, reps, best, ms_best, ms_default)) return -1;
+    c->adapt = false;
+    if (rebuild(start.adapt ? &ms_end : nullptr)) return -1;
+    if (!start.adapt) return 0;
+    ms_default = ms_start;
+    ms_best = ms_end;
+    if (ms_end < 0.99 * ms_start && !(b->prec == SP3MM_PREC_MIXED && same_tuning(best, start.tune))) return 0;
+    c->tune = best = start.tune;
+    c->adapt = true;
+    ms_best = ms_start;
+    return rebuild(nullptr);
 }
 
 // Copies the current entries of the batch's operands (the same count, shapes
