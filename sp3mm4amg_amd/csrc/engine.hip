@@ -783,16 +783,17 @@ static int spgemm_onepass(const sp3mm_dmat &A, const sp3mm_dmat &B, sp3mm_dmat &
     }
     Ctl *d = ctl.as<Ctl>();
     Ctl h;
-    // Bins of at most kSpgMergeRows rows fold into the next larger one (a launch
-    // of 8 boundary rows took 8 us and its gather 5; folded rows take a larger
-    // slot each, 200 MB in all at most), and the host polls for the populations.
+    // Bins of at most kSpgMergeRows rows fold into one up to four times as large
+    // (a launch of 8 boundary rows took 8 us and its gather 5; folded rows take
+    // larger slots and as much more of the output's arrays), and the host polls
+    // for the populations.
     // The binning clears the control block (there is none without rows).
     // Pair product of a 7-point 80^3 operator: 458 -> 423 us.
     const unsigned long long seq = c->poll_host && M > 0 ? ++c->poll_seq : 0;
     if (M == 0) launch_fill_i32(reinterpret_cast<int32_t *>(d), (int64_t)(sizeof(Ctl) / 4), 0, s);
     SP3MM_HIP(hipGetLastError());
     launch_ub_bin(a, b, ub.as<int64_t>(), rown.as<int32_t>(), lists.as<int32_t>(), d->rawc, thr, d->totals,
-                  binscr.as<int>(), s, kSpgMergeRows, d->counts, d, seq ? c->poll_dev : nullptr,
+                  binscr.as<int>(), s, MergeRule{0, kSpgMergeRows}, d->counts, d, seq ? c->poll_dev : nullptr,
                   (int)(sizeof(Ctl) / 4),
                   seq ? reinterpret_cast<unsigned long long *>(c->poll_dev + kPollFlagOff) : nullptr, seq, 0, nullptr,
                   -1, 0, false, nullptr, M > 0 && A.nnz >= (int64_t)kWaveUbRow * M);
@@ -1423,14 +1424,16 @@ struct FusedPlan {
         }
     }
 
-    // Bins of at most kMergeRows rows are folded into the next larger non-empty
-    // bin while the binning writes its lists (its tables hold their upper
-    // bounds too): a launch that does not fill the chip once (256 CUs x 24
-    // wavefronts) costs a whole row's latency, while the appended rows fill
-    // groups of the larger launch.  27-point 100^3 product: its 3464 boundary
-    // rows took 71 us behind the other 35840 as a launch of their own.
+    // Small bins are folded into the next larger non-empty bin while the
+    // binning writes its lists (its tables hold their upper bounds too): a
+    // launch that does not fill the chip once (256 CUs x 24 wavefronts) costs a
+    // whole row's latency, while the appended rows fill groups of the larger
+    // launch.  27-point 100^3 product: its 3464 boundary rows took 71 us behind
+    // the other 35840 as a launch of their own.  More than kMergeAny rows only
+    // into tables of about their size (MergeRule), and not in the
+    // allocation-free product, whose scratch their larger slots could exceed.
     // d()->counts holds the merged populations, d()->rawc those before.
-    static constexpr int kMergeRows = 8192;
+    static constexpr int kMergeAny = 1024, kMergeNearRows = 8192;
 
     // The binning clears the control block first; with seq > 0 its scatter
     // kernel also exports the block to the coherent host block with that
@@ -1454,7 +1457,8 @@ struct FusedPlan {
             ob.word = (int)(offsetof(Ctl, onebin) / 4);
         }
         launch_ub_bin(r(), a(), ub.as<int64_t>(), rown.as<int32_t>(), lists.as<int32_t>(), d()->rawc, thr,
-                      d()->totals, binscr.as<int>(), s, kMergeRows, d()->counts, d(), host,
+                      d()->totals, binscr.as<int>(), s,
+                      MergeRule{kMergeAny, ext_out ? kMergeAny : kMergeNearRows}, d()->counts, d(), host,
                       (int)(sizeof(Ctl) / 4), flag, seq, span_lim, &d()->pred_count, pred, big_from,
                       reassoc_possible(c), one ? &ob : nullptr, R.M > 0 && R.nnz >= (int64_t)kWaveUbRow * R.M);
     }

@@ -420,13 +420,13 @@ __global__ void __launch_bounds__(1024) k_bin_offsets(int *__restrict__ hist, in
     }
 }
 
-// Bins of at most `lim` rows fold into the next larger non-empty hash bin
+// Bins of few rows (MergeRule) fold into the next larger non-empty hash bin
 // (a launch of a handful of rows costs a whole row's latency, while appended
 // rows fill groups of the larger launch; chains of small bins move up
 // together).  From the bin populations raw[0..nb]: dest[b] is the bin whose
 // list takes bin b's rows, starting at position start[b]; cnt[b] the merged
 // populations.  The long bin nb never merges.
-__device__ __forceinline__ void merge_plan(const int *raw, int nb, int lim, int *dest, int *start, int *cnt)
+__device__ __forceinline__ void merge_plan(const int *raw, int nb, MergeRule rule, int *dest, int *start, int *cnt)
 {
     for (int b = 0; b <= nb; b++) {
         cnt[b] = raw[b];
@@ -434,10 +434,13 @@ __device__ __forceinline__ void merge_plan(const int *raw, int nb, int lim, int 
         start[b] = 0;
     }
     for (int b = 0; b < nb; b++) {
-        if (cnt[b] == 0 || cnt[b] > lim) continue;
-        int to = b + 1;
+        if (cnt[b] == 0 || cnt[b] > max(rule.any, rule.near)) continue;
+        int to = b + 1, low = b;  // low: the smallest bin whose rows are here
         while (to < nb && cnt[to] == 0) to++;
         if (to >= nb) continue;
+        for (int c = b; c >= 0; c--)
+            if (dest[c] == b && raw[c] > 0) low = c;
+        if (cnt[b] > rule.any && to - low > kMergeNear) continue;
         for (int c = 0; c <= b; c++)
             if (dest[c] == b) {
                 dest[c] = to;
@@ -448,7 +451,7 @@ __device__ __forceinline__ void merge_plan(const int *raw, int nb, int lim, int 
     }
 }
 
-// merge_lim > 0: rows land in their merged bins (merge_plan over the
+// merge.near > 0: rows land in their merged bins (merge_plan over the
 // populations `raw` that k_bin_offsets produced), and workgroup 0 writes the
 // merged populations to `mcounts`
 // ex (optional): workgroup 0 also exports the control block ex.src (bin
@@ -478,7 +481,7 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_scatter(const int64_t *__re
                                                               const int32_t *__restrict__ meas2, int64_t M,
                                                               const int *__restrict__ hist, int32_t *__restrict__ lists,
                                                               BinThresholds thr, const int *__restrict__ raw,
-                                                              int merge_lim, int *__restrict__ mcounts, CtlExport ex)
+                                                              MergeRule merge, int *__restrict__ mcounts, CtlExport ex)
 {
     __shared__ int h[kMaxBins + 1];
     // the merge plan in LDS (indexed by bin: no private-memory arrays)
@@ -494,15 +497,15 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_scatter(const int64_t *__re
     // in one-bin mode only workgroup 0 needs the plan (for the populations
     // it publishes); the others list their rows in row order
     if (threadIdx.x == 0 && (sone_sh == 0 || blockIdx.x == 0)) {
-        if (merge_lim > 0) {
-            merge_plan(raw, thr.nb, merge_lim, mdest, mstart, cnt);
+        if (merge.near > 0) {
+            merge_plan(raw, thr.nb, merge, mdest, mstart, cnt);
         } else {
             for (int b = 0; b < nbin; b++) {
                 mdest[b] = b;
                 mstart[b] = 0;
             }
         }
-        if (merge_lim > 0 && blockIdx.x == 0)
+        if (merge.near > 0 && blockIdx.x == 0)
             for (int b = 0; b < nbin; b++) mcounts[b] = cnt[b];
         if (ex.pred_count && blockIdx.x == 0) {
             bool reassoc = false;
@@ -511,7 +514,7 @@ __global__ void __launch_bounds__(kBinThreads) k_bin_scatter(const int64_t *__re
                 for (int b = ex.big_from; b < nbin; b++) big += raw[b];
                 reassoc = 2 * big >= M && 2 * (long long)ex.totals[2] >= M;
             }
-            *ex.pred_count = reassoc || ex.pred < 0 ? 0 : (merge_lim > 0 ? cnt[ex.pred] : raw[ex.pred]);
+            *ex.pred_count = reassoc || ex.pred < 0 ? 0 : (merge.near > 0 ? cnt[ex.pred] : raw[ex.pred]);
         }
     }
     __syncthreads();
@@ -2408,7 +2411,7 @@ int64_t bin_scratch_ints(int64_t M) { return (kMaxBins + 1) * ((M + kBinThreads 
 
 static void launch_bins(const SpOperand *A, const SpOperand *B, const int32_t *m1, const int32_t *m2, int64_t M,
                         int64_t *ub, int32_t *rownnz, int32_t *lists, int *counts, const BinThresholds &thr,
-                        unsigned long long *totals, int *scratch, hipStream_t st, int merge_lim = 0,
+                        unsigned long long *totals, int *scratch, hipStream_t st, MergeRule merge = {},
                         int *mcounts = nullptr, const CtlExport *ex = nullptr, const OneBin *one = nullptr,
                         bool wave_ub = false)
 {
@@ -2445,12 +2448,12 @@ static void launch_bins(const SpOperand *A, const SpOperand *B, const int32_t *m
     CtlExport e{};
     if (ex) e = *ex;
     hipLaunchKernelGGL(k_bin_scatter, dim3(nblk), dim3(kBinThreads), 0, st, ub, m1, m2, M, hist, lists, thr, counts,
-                       merge_lim, mcounts, e);
+                       merge, mcounts, e);
 }
 
 void launch_ub_bin(const SpOperand &A, const SpOperand &B, int64_t *ub, int32_t *rownnz,
                    int32_t *lists, int *counts, const BinThresholds &thr,
-                   unsigned long long *totals, int *scratch, hipStream_t st, int merge_lim, int *mcounts,
+                   unsigned long long *totals, int *scratch, hipStream_t st, MergeRule merge, int *mcounts,
                    const void *ctl, void *ctl_host, int ctl_words, unsigned long long *flag, unsigned long long seq,
                    int span_lim, int *pred_count, int pred, int big_from, bool reassoc_possible, const OneBin *one,
                    bool wave_ub)
@@ -2458,7 +2461,7 @@ void launch_ub_bin(const SpOperand &A, const SpOperand &B, int64_t *ub, int32_t 
     CtlExport e{static_cast<const uint32_t *>(ctl), static_cast<uint32_t *>(ctl_host), ctl_words, flag, seq,
                 ctl != nullptr, span_lim, pred_count, pred, big_from, reassoc_possible, totals,
                 ctl && one ? one->word : -1};
-    launch_bins(&A, &B, nullptr, nullptr, A.M, ub, rownnz, lists, counts, thr, totals, scratch, st, merge_lim,
+    launch_bins(&A, &B, nullptr, nullptr, A.M, ub, rownnz, lists, counts, thr, totals, scratch, st, merge,
                 mcounts, ctl ? &e : nullptr, ctl ? one : nullptr, wave_ub);
 }
 
