@@ -48,10 +48,10 @@ def test_products_around_the_rule(short, short_len, long, long_len):
 
 
 def test_allocation_free_product_keeps_small_slots():
-    """8,000 rows of 7 products and 2,600 of 4,900: in slots of the long rows'
+    """8,000 rows of 7 products and 3,100 of 4,900: in slots of the long rows'
     size they need more than the 256 MB of fixed scratch."""
     L.set_tuning(None)
-    ops = _operands(8000, 1, 2600, 700)
+    ops = _operands(8000, 1, 3100, 700)
     d = [L.DeviceCSR.upload(m) for m in ops]
     ref, _ = L.rap(*d)
     want = ref.download()
