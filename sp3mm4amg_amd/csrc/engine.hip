@@ -41,6 +41,12 @@ size_t Pool::size_class(size_t b)
     return (b + g - 1) / g * g;
 }
 
+hipError_t Pool::fresh(void **p, size_t c) const
+{
+    if (limit && held_ + cached_ + c > limit) return hipErrorOutOfMemory;
+    return hipMalloc(p, c);
+}
+
 void *Pool::alloc(size_t bytes)
 {
     const size_t c = size_class(bytes ? bytes : 1);
@@ -50,26 +56,26 @@ void *Pool::alloc(size_t bytes)
         void *p = it->second;
         free_.erase(it);
         cached_ -= c;
+        held_ += c;
         live_[p] = c;
         return p;
     }
     void *p = nullptr;
-    hipError_t e = hipMalloc(&p, c);
+    hipError_t e = fresh(&p, c);
     if (e != hipSuccess) {
         (void)hipGetLastError();
         for (auto &kv : free_) (void)hipFree(kv.second);
         free_.clear();
         cached_ = 0;
-        e = hipMalloc(&p, c);
+        e = fresh(&p, c);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            size_t live = 0;
-            for (auto &kv : live_) live += kv.second;
             set_error("hipMalloc(%zu) failed: %s (library holds %zu bytes in %zu live blocks)", c,
-                      hipGetErrorString(e), live, live_.size());
+                      hipGetErrorString(e), held_, live_.size());
             return nullptr;
         }
     }
+    held_ += c;
     live_[p] = c;
     return p;
 }
@@ -82,6 +88,7 @@ void Pool::release(void *p)
     if (it == live_.end()) return;
     free_.emplace(it->second, p);
     cached_ += it->second;
+    held_ -= it->second;
     live_.erase(it);
 }
 
@@ -182,6 +189,7 @@ int init_device(int dev)
         const size_t v = (size_t)strtoull(cap, nullptr, 10);
         if (v >= 16384 && v < c->max_lds) c->max_lds = v;
     }
+    if (const char *v = getenv("SP3MM_POOL_LIMIT")) c->pool.limit = (size_t)strtoull(v, nullptr, 10);
     tuning_from_env(c->tune);
     c->adapt = same_tuning(c->tune, Tuning{});
     SP3MM_HIP(hipStreamCreateWithFlags(&c->own_stream, hipStreamNonBlocking));
@@ -1209,13 +1217,27 @@ static int likely_bin(const BinThresholds &thr, const sp3mm_dmat &R, const sp3mm
 // counters back to size bins, scratch slots and the output; record() enqueues
 // the same kernels for the sizes found by build() with no host
 // synchronisation, so it can be captured into a HIP graph and replayed.
-struct FusedPlan {
+struct PlanInput {
     sp3mm_dmat R{}, A{}, P{};
     bool mixed = false;  // FP32-pair accumulation kernel
     bool f32 = false;    // FP32 operands (mixed, or FP64 accumulation of FP32 inputs)
     double guard = 1e-2;
     double *rowsum = nullptr;
     Tuning tu{};
+    // per-phase device times (ms_ub, ms_num, ms_scan): HIP events between the
+    // phases, which add gaps to the stream; off unless asked for
+    bool detail = false;
+    // choose the tables' sizes and multipliers from a sample of R's rows
+    // (large products whose schedule nobody set)
+    bool adapt = false;
+    bool keep = false;  // the plan will be replayed: sample every bin of it, whatever the product's size
+    // One-off FP64 products may be reassociated: build() stops after the
+    // binning and sets `reassoc` when most rows are beyond the one-wavefront
+    // tables and the output is wider than an LDS window (the caller then runs
+    // R*(A*P) as two SpGEMMs; see wants_reassoc)
+    bool reassoc_ok = false;
+};
+struct FusedPlan : PlanInput {
     BinThresholds thr{};
     std::vector<FusedCfg> cfg;
     std::vector<int> cnt, fcnt;
@@ -1232,20 +1254,10 @@ struct FusedPlan {
     // output and keeps no long-row slots (scratch comes from an Arena).
     bool ext_out = false;
     int64_t ext_cap = 0;
-    // per-phase device times (ms_ub, ms_num, ms_scan): HIP events between the
-    // phases, which add gaps to the stream; off unless asked for
-    bool detail = false;
     int mk(Timer &tm) const { return detail ? tm.mark() : -1; }
-    // Choose the tables' sizes and multipliers from a sample of R's rows
-    // (large products whose schedule nobody set); sampled: build() did
-    bool adapt = false, sampled = false;
-    bool keep = false;  // the plan will be replayed: sample every bin of it, whatever the product's size
+    bool sampled = false;  // build() adapted the tables
     int big_from = 0;  // first bin of multi-wavefront groups under the plan's schedule
-    // One-off FP64 products may be reassociated: build() stops after the
-    // binning and sets `reassoc` when most rows are beyond the one-wavefront
-    // tables and the output is wider than an LDS window (the caller then runs
-    // R*(A*P) as two SpGEMMs; see wants_reassoc)
-    bool reassoc_ok = false, reassoc = false;
+    bool reassoc = false;
 
     // (re)allocates the output arrays for `cap` entries
     int alloc_out(Context *c, int64_t cap)
@@ -1990,6 +2002,22 @@ struct FusedPlan {
     }
 };
 
+// plan.build().  Slots for sampled tables, and the dense ones of unmerged rows
+// (up to 4 GiB), can take memory that the schedule's own tables do without: an
+// adapted plan that fails is built once more as its schedule stands.
+static int build_plan(Context *c, FusedPlan &plan, Timer &tm)
+{
+    PlanInput in = plan;
+    if (plan.build(c, tm) == 0) return 0;
+    if (!in.adapt) return -1;
+    plan.release_all();
+    plan = FusedPlan();
+    in.adapt = false;
+    static_cast<PlanInput &>(plan) = in;
+    clear_error();
+    return plan.build(c, tm);
+}
+
 static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, sp3mm_dmat &C,
                             sp3mm_stats *st, int prec, double guard, double *rowsum, bool timing)
 {
@@ -2008,7 +2036,7 @@ static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3m
     plan.reassoc_ok = prec == SP3MM_PREC_FP64 && !rowsum;
     plan.detail = timing;
     plan.adapt = c->adapt;
-    if (plan.build(c, tm)) {
+    if (build_plan(c, plan, tm)) {
         plan.release_all();
         return -1;
     }
@@ -3140,7 +3168,7 @@ static int batch_build(Context *c, Batch *b, bool graph)
     b->plan.adapt = c->adapt;
     b->plan.keep = true;
     b->plan.guard = b->guard;
-    if (b->plan.build(c, tm)) return -1;
+    if (build_plan(c, b->plan, tm)) return -1;
     b->export_bounds(c->stream);
     const int e2 = tm.mark();
     (void)hipEventSynchronize(tm.ev[e2]);
@@ -3684,7 +3712,7 @@ void *hier_create(const sp3mm_dmat &A, int nlev, const int64_t *const *aggs, con
         L.rap.tu = c->tune;
         L.rap.adapt = c->adapt;
         L.rap.keep = true;
-        if (L.rap.build(c, t2)) {
+        if (build_plan(c, L.rap, t2)) {
             hier_release(h);
             return nullptr;
         }

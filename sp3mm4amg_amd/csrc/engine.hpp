@@ -27,9 +27,11 @@ void clear_error();
 
 // Caching allocator: blocks are rounded up to a size class (at most 1/8 waste)
 // and kept on per-class free lists for reuse; everything is released when a
-// fresh hipMalloc fails.
+// fresh hipMalloc fails, or would take the blocks held beyond `limit` bytes
+// (SP3MM_POOL_LIMIT; 0: as much as the device has).
 class Pool {
   public:
+    size_t limit = 0;
     void *alloc(size_t bytes);
     void release(void *p);
     void trim();
@@ -37,9 +39,10 @@ class Pool {
 
   private:
     static size_t size_class(size_t bytes);
+    hipError_t fresh(void **p, size_t c) const;
     std::multimap<size_t, void *> free_;
     std::map<void *, size_t> live_;
-    size_t cached_ = 0;
+    size_t cached_ = 0, held_ = 0;  // bytes on the free lists, in live blocks
     std::mutex mu_;
 };
 
