@@ -432,7 +432,7 @@ struct Ctl {
     unsigned long long totals[3];  // bound sum, bound maximum, rows of unstructured spread
     int64_t nnz;
     int longest;  // longest row seen (prolongator)
-    int pad2;
+    int nagain;   // rows whose tables filled under the schedule's sizes, too (run_again)
 };
 
 static int max_blocks(const Context *c) { return c->num_cu * 16; }
@@ -1256,6 +1256,13 @@ struct FusedPlan : PlanInput {
     int64_t ext_cap = 0;
     int mk(Timer &tm) const { return detail ? tm.mark() : -1; }
     bool sampled = false;  // build() adapted the tables
+    std::vector<FusedCfg> unsampled;  // cfg under the schedule's own sizes, then
+    // Rows whose sampled tables filled, run once more (run_again): their list
+    // and slots of again_h2 entries.  `retry` then holds the rows that filled
+    // those tables as well, counted by Ctl::nagain.
+    Buf again, aslotn, acol, aval;
+    int nagain = 0, again_h2 = 0;
+    int *retry_count() const { return nagain ? &d()->nagain : &d()->nretry; }
     int big_from = 0;  // first bin of multi-wavefront groups under the plan's schedule
     bool reassoc = false;
 
@@ -1376,6 +1383,10 @@ struct FusedPlan : PlanInput {
                                (int)(sizeof(Ctl) / 4));
             exported = exported || x;
         }
+        if (nagain)
+            launch_gather_rows(again.as<int32_t>(), &d()->nretry, nagain, aslotn.as<int32_t>(), again_h2,
+                               acol.as<int32_t>(), aval.as<double>(), C.rp, C.col, static_cast<double *>(C.val), ccap,
+                               &d()->err, max_blocks(c), s);
         launch_long(c, s, true);
         return exported;
     }
@@ -1414,7 +1425,7 @@ struct FusedPlan : PlanInput {
                                  num ? C.col : nullptr, cv, rs, cap, &d()->err, s, f32);
         }
         if (!defer_retry && (nretry > 0 || (!num && !built) || (num && spec)))
-            launch_window_direct(num, c->num_cu, wl, r(), a(), p(), retry.as<int32_t>(), &d()->nretry, dlog1,
+            launch_window_direct(num, c->num_cu, wl, r(), a(), p(), retry.as<int32_t>(), retry_count(), dlog1,
                                  spill.as<int32_t>(), &d()->nspill, rn, num ? C.rp : nullptr, num ? C.col : nullptr,
                                  cv, rs, cap, &d()->err, s, f32);
         if (nspill > 0)
@@ -1567,8 +1578,44 @@ struct FusedPlan : PlanInput {
         // scratch slots beyond both the schedule's own and 4 GiB are not worth it
         if (slots > cfg[pred].H2 && R.M * slots * 12 > ((int64_t)4 << 30)) return false;
         for (FusedCfg &g : f) take_multipliers(g, so);
+        unsampled = std::move(cfg);
         cfg = f;
         return true;
+    }
+
+    // The rows whose sampled tables filled (nretry of them), in tables of the
+    // bound of the largest bin at hand, so that no more rows are redone by the
+    // long-row kernels than without the sample.  They are few, so a row gets a
+    // wavefront or more, and a stage-2 table as large as stage 1's where LDS
+    // holds both (one of 64 slots for 60 keys took 97 us for 133 rows).  40,000
+    // rows of 20 x 9 products, 133 of them scattered over 160,000 columns, which
+    // the long-row kernels take one by one in HBM: 143 us unsampled, 340 when
+    // the sample missed the 133, 224 this way.
+    void run_again(Context *c, hipStream_t s)
+    {
+        int b = thr.nb - 1;
+        while (b > 0 && cnt[b] == 0) b--;
+        FusedCfg f = unsampled[b];
+        f.G = f.H1 <= 512 ? 64 : 256;
+        const int least = std::max(f.H2, f.G);
+        for (f.H2 = std::max(f.H1, f.G); f.H2 > least && fused_lds(f.G, f.H1, f.H2) > c->max_lds; f.H2 /= 2) {
+        }
+        if (fused_lds(f.G, f.H1, f.H2) > c->max_lds) return;
+        Buf list((size_t)nretry * 4);
+        aslotn = Buf((size_t)nretry * 4);
+        acol = Buf((size_t)nretry * f.H2 * 4);
+        aval = Buf((size_t)nretry * f.H2 * 8);
+        if (!list.p || !aslotn.p || !acol.p || !aval.p) {
+            clear_error();
+            return;
+        }
+        launch_direct_fused(f.G, f.H1, f.H2, slog1, slog2, r(), a(), p(), retry.as<int32_t>(), &d()->nretry, nretry,
+                            rown.as<int32_t>(), aslotn.as<int32_t>(), acol.as<int32_t>(), aval.as<double>(),
+                            list.as<int32_t>(), &d()->nagain, &d()->err, max_blocks(c), s, f32, tu);
+        again = std::move(retry);
+        retry = std::move(list);
+        nagain = nretry;
+        again_h2 = f.H2;
     }
 
     // Forwarding without merging (k_scatter_direct) for the rows of
@@ -1899,12 +1946,13 @@ struct FusedPlan : PlanInput {
             if (h.nretry > 0) {
                 // the retried rows' lengths (window count pass), then the scan again
                 nretry = h.nretry;
+                if (sampled && !keep) run_again(c, s);
                 launch_long(c, s, false);
                 launch_scan(rown.as<int32_t>(), M, C.rp, C.rp32, tiles.as<long long>(), &d()->nnz, s);
             }
         }
         if (read_ctl(c, d(), h)) return -1;
-        nretry = h.nretry;
+        nretry = nagain ? h.nagain : h.nretry;
         nspill = h.nspill;
         nwide = h.nwide;
         built = true;
@@ -2004,11 +2052,14 @@ struct FusedPlan : PlanInput {
 
 // plan.build().  Slots for sampled tables, and the dense ones of unmerged rows
 // (up to 4 GiB), can take memory that the schedule's own tables do without: an
-// adapted plan that fails is built once more as its schedule stands.
+// adapted plan that fails is built once more as its schedule stands.  So is one
+// to be replayed with rows that its sampled tables do not hold: every replay
+// would run them on the long-row kernels.
 static int build_plan(Context *c, FusedPlan &plan, Timer &tm)
 {
     PlanInput in = plan;
-    if (plan.build(c, tm) == 0) return 0;
+    const int rc = plan.build(c, tm);
+    if (rc == 0 && !(plan.keep && plan.sampled && plan.nretry > 0)) return 0;
     if (!in.adapt) return -1;
     plan.release_all();
     plan = FusedPlan();
