@@ -532,11 +532,14 @@ struct Timer {
     }
 };
 
-// the coherent block: the control block at 0, the sample of rows behind it,
-// and the sequence flags of both at its end
+// the coherent block: the control block at 0, the sample of rows and the
+// consumers' state behind it, and the sequence flags of the three at its end
 constexpr size_t kPollFlagOff = 4088;
 constexpr size_t kSampleOff = 2048, kSampleFlagOff = 4080;
-static_assert(sizeof(Ctl) <= kSampleOff && kSampleOff + sizeof(SampleOut) <= kSampleFlagOff, "the parts do not overlap");
+constexpr size_t kConsOff = 4032, kConsFlagOff = 4072;
+static_assert(sizeof(Ctl) <= kSampleOff && kSampleOff + sizeof(SampleOut) <= kConsOff &&
+                  kConsOff + sizeof(ConsState) <= kConsFlagOff,
+              "the parts do not overlap");
 
 template <typename Query, typename Block>
 static hipError_t spin_wait(Query q, Block b)
@@ -579,7 +582,7 @@ static int wait_flag(Context *c, size_t off, unsigned long long seq)
             const hipError_t q = hipStreamQuery(c->stream);
             if (q == hipSuccess) {
                 if (__atomic_load_n(flag_host, __ATOMIC_ACQUIRE) == seq) break;
-                set_error("control block export did not arrive (sequence %llu)", seq);
+                set_error("an export to the host did not arrive (sequence %llu)", seq);
                 return -1;
             }
             if (q != hipErrorNotReady) {
@@ -2559,13 +2562,15 @@ int consumer_wait(Context *c, double *dot_out)
     }
     ConsState h{};
     static_assert(sizeof(ConsState) % 4 == 0, "exported as words");
-    if (c->host_small_dev) {
-        // a copy into pageable memory and a blocking wait left the GPU idle
-        // for 37 us between the cycles of a solve
-        launch_export_words(c->cons, c->host_small_dev, (int)(sizeof h / 4), c->stream);
-        SP3MM_HIP(hipGetLastError());
-        SP3MM_HIP(spin_stream(c->stream));
-        memcpy(&h, c->host_small, sizeof h);
+    if (c->poll_host) {
+        // a copy into pageable memory and a blocking wait left the GPU idle for
+        // 37 us between the cycles of a solve; an export and stream queries took
+        // 37 to 45 us behind a single sweep, where the copy took 30 and this takes 18
+        const unsigned long long seq = ++c->poll_seq;
+        launch_export_flag(c->cons, c->poll_dev + kConsOff, (int)(sizeof h / 4),
+                           reinterpret_cast<unsigned long long *>(c->poll_dev + kConsFlagOff), seq, c->stream);
+        if (wait_flag(c, kConsFlagOff, seq)) return -1;
+        memcpy(&h, c->poll_host + kConsOff, sizeof h);
     } else {
         SP3MM_HIP(hipMemcpyAsync(&h, c->cons, sizeof h, hipMemcpyDeviceToHost, c->stream));
         SP3MM_HIP(hipStreamSynchronize(c->stream));

@@ -2389,6 +2389,18 @@ __global__ void k_export_words(const uint32_t *__restrict__ src, uint32_t *dst, 
     for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
 }
 
+// the same into coherent host memory, and then *flag = seq: the host polls that
+// word instead of asking for the stream's state
+__global__ void __launch_bounds__(64) k_export_flag(const uint32_t *__restrict__ src, uint32_t *dst, int n,
+                                                    unsigned long long *flag, unsigned long long seq)
+{
+    for (int i = threadIdx.x; i < n; i += 64)
+        __hip_atomic_store(dst + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flag, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3629,6 +3641,13 @@ void launch_export_words(const void *src, void *host_dst, int words, hipStream_t
 {
     hipLaunchKernelGGL(k_export_words, dim3(1), dim3(64), 0, st, static_cast<const uint32_t *>(src),
                        static_cast<uint32_t *>(host_dst), words);
+}
+
+void launch_export_flag(const void *src, void *host_dst, int words, unsigned long long *flag, unsigned long long seq,
+                        hipStream_t st)
+{
+    hipLaunchKernelGGL(k_export_flag, dim3(1), dim3(64), 0, st, static_cast<const uint32_t *>(src),
+                       static_cast<uint32_t *>(host_dst), words, flag, seq);
 }
 
 void launch_fill_i32(int32_t *p, int64_t n, int32_t v, hipStream_t st)

@@ -329,6 +329,8 @@ int dot_parts();
 void launch_jacobi(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz, const double *b,
                    const double *xi, double *xo, double omega, int *err, hipStream_t st);
 void launch_export_words(const void *src, void *host_dst, int words, hipStream_t st);
+void launch_export_flag(const void *src, void *host_dst, int words, unsigned long long *flag, unsigned long long seq,
+                        hipStream_t st);
 void launch_copy_probe(const void *in, void *out, int64_t bytes, hipStream_t st);
 
 }  // namespace sp3mm
