@@ -116,7 +116,7 @@ int sp3mm_dmat_upload(sp3mm_dmat *out, int64_t M, int64_t N, int64_t nnz, const 
                   (long long)irp[0], (long long)irp[M], (long long)nnz);
         return -1;
     }
-    if (host_io_fits(M, nnz, vtype)) {
+    if (host_io_fits(M, nnz, vtype, ja, val)) {
         const int rc = upload_large(out, M, N, nnz, irp, ja, val, vtype, base);
         if (rc <= 0) return rc;
     }
@@ -271,7 +271,7 @@ int sp3mm_dmat_download(const sp3mm_dmat *m, int64_t *irp, int64_t *ja, void *va
     std::lock_guard<std::recursive_mutex> lk(c->mu);
     hipStream_t s = c->stream;
     const int64_t M = m->M, nnz = m->nnz;
-    if (ja && val && host_io_fits(M, nnz, m->vtype)) {
+    if (ja && val && host_io_fits(M, nnz, m->vtype, ja, val)) {
         const int rc = host_download(c, *m, irp, ja, val, base);
         if (rc <= 0) return rc;
     }

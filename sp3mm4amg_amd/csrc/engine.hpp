@@ -112,7 +112,7 @@ struct HostCheck {
     int64_t bad_row = -1;  // first row whose offsets decrease
     bool bad_col = false;  // a column out of range
 };
-bool host_io_fits(int64_t M, int64_t nnz, int vtype);
+bool host_io_fits(int64_t M, int64_t nnz, int vtype, const int64_t *ja, const void *val);
 int host_upload(Context *c, const sp3mm_dmat &m, const int64_t *irp, const int64_t *ja, const void *val, int base,
                 HostCheck &chk);
 int host_download(Context *c, const sp3mm_dmat &m, int64_t *irp, int64_t *ja, void *val, int base);

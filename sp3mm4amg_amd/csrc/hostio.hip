@@ -174,10 +174,26 @@ bool ring_ready(Context *c)
 constexpr size_t kMinBytes = (size_t)6 << 20;
 }  // namespace
 
-bool host_io_fits(int64_t M, int64_t nnz, int vtype)
+// memory the runtime knows nothing of, which it would stage itself
+static bool pageable(const void *p)
+{
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
+// Arrays in pinned memory are not staged: one copy of each runs at the bus's
+// rate, and the pages of a new array are not touched from the host.  7-point
+// operators, up / down in ms: 48^3 0.32 / 0.28 against 0.41 / 0.34 staged, 96^3
+// 2.15 / 1.91 against 2.15 / 1.80, and into new pinned arrays 1.9 against 9 to 12.
+bool host_io_fits(int64_t M, int64_t nnz, int vtype, const int64_t *ja, const void *val)
 {
     return nnz < INT32_MAX &&
-           (size_t)(M + 1) * 8 + (size_t)nnz * (8 + (vtype == SP3MM_F32 ? 4 : 8)) >= kMinBytes;
+           (size_t)(M + 1) * 8 + (size_t)nnz * (8 + (vtype == SP3MM_F32 ? 4 : 8)) >= kMinBytes &&
+           (pageable(ja) || pageable(val));
 }
 
 int host_upload(Context *c, const sp3mm_dmat &m, const int64_t *irp, const int64_t *ja, const void *val, int base,
