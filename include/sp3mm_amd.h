@@ -252,6 +252,11 @@ int sp3mm_init(int device);
 const char *sp3mm_last_error(void);
 /* Block until all queued device work of the library has finished. */
 int sp3mm_sync(void);
+/* Waits like sp3mm_sync and gives back what the library keeps for later calls
+ * and nothing uses at the time: device blocks of its pool, and the 16 MB of
+ * pinned staging that large host copies share (each is taken again by the next
+ * call that needs it). */
+int sp3mm_trim(void);
 /* Queue the library's device work on the caller's HIP stream (a hipStream_t
  * created by the caller, not the null stream; NULL restores the library's own
  * stream).  Work already queued on the previous stream finishes first.  Calls

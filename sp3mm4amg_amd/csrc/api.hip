@@ -51,6 +51,18 @@ int sp3mm_sync(void)
     return consumer_wait(c);
 }
 
+int sp3mm_trim(void)
+{
+    clear_error();
+    Context *c = ctx();
+    if (!c) return -1;
+    std::lock_guard<std::recursive_mutex> lk(c->mu);
+    SP3MM_HIP(hipStreamSynchronize(c->stream));
+    c->pool.trim();
+    ring_release(c);
+    return 0;
+}
+
 static void set_not_csr(int base)
 {
     set_error("upload: matrix is not valid sorted CSR (offsets must be monotone from %d to "

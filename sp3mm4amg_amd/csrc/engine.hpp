@@ -46,8 +46,8 @@ class Pool {
     std::mutex mu_;
 };
 
-// Pinned staging of large host copies (16 MB, allocated by the first one), and
-// an event per group of slots.
+// Pinned staging of large host copies (16 MB, allocated by the first one and
+// given back by sp3mm_trim), and an event per group of slots.
 struct HostRing {
     unsigned char *mem = nullptr;
     unsigned char *dev = nullptr;  // its device-side address
@@ -113,6 +113,7 @@ struct HostCheck {
     bool bad_col = false;  // a column out of range
 };
 bool host_io_fits(int64_t M, int64_t nnz, int vtype, const int64_t *ja, const void *val);
+void ring_release(Context *c);
 int host_upload(Context *c, const sp3mm_dmat &m, const int64_t *irp, const int64_t *ja, const void *val, int base,
                 HostCheck &chk);
 int host_download(Context *c, const sp3mm_dmat &m, int64_t *irp, int64_t *ja, void *val, int base);

@@ -144,6 +144,13 @@ bool aligned16(const sp3mm_dmat &m)
              reinterpret_cast<uintptr_t>(m.val)) & 15) == 0;
 }
 
+void drop_ring(HostRing *r)
+{
+    for (auto e : r->ev) (void)hipEventDestroy(e);
+    if (r->mem) (void)hipHostFree(r->mem);
+    delete r;
+}
+
 bool ring_ready(Context *c)
 {
     if (c->ring) return true;
@@ -159,9 +166,7 @@ bool ring_ready(Context *c)
     }
     if (!ok) {
         (void)hipGetLastError();
-        for (auto e : r->ev) (void)hipEventDestroy(e);
-        if (r->mem) (void)hipHostFree(r->mem);
-        delete r;
+        drop_ring(r);
         return false;
     }
     c->ring = r;
@@ -173,6 +178,13 @@ bool ring_ready(Context *c)
 // ms this way and 1.02 pageable; 48^3, 7 to 13 MB, 1.26 and 1.63).
 constexpr size_t kMinBytes = (size_t)6 << 20;
 }  // namespace
+
+// under the context's lock, behind its stream
+void ring_release(Context *c)
+{
+    if (c->ring) drop_ring(c->ring);
+    c->ring = nullptr;
+}
 
 // memory the runtime knows nothing of, which it would stage itself
 static bool pageable(const void *p)

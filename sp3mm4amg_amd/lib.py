@@ -182,6 +182,7 @@ def lib():
         L.sp3mm_hier_free.argtypes = [C.c_void_p]
         L.sp3mm_hier_free.restype = None
         L.sp3mm_sync.restype = C.c_int
+        L.sp3mm_trim.restype = C.c_int
         L.sp3mm_set_stream.argtypes = [C.c_void_p]
         L.sp3mm_get_stream.restype = C.c_void_p
         L.sp3mm_copy_probe.argtypes = [C.c_int64, C.c_int32]
@@ -575,6 +576,11 @@ def get_stream() -> int | None:
 def sync() -> None:
     """Waits for the library's stream; raises on an error a queued call left."""
     _check(lib().sp3mm_sync(), "sp3mm_sync")
+
+
+def trim() -> None:
+    """Gives back the device and pinned memory kept for later calls."""
+    _check(lib().sp3mm_trim(), "sp3mm_trim")
 
 
 def dot(x: DeviceArray, y: DeviceArray) -> float:
