@@ -451,7 +451,9 @@ int sp3mm_get_tuning(sp3mm_tuning *t);
  * this call, the autotuner or the environment), the FP64 and MIXED64 direct
  * products, batches and hierarchies adapt the table sizes, group widths and
  * hash multipliers to a sample of the operands' rows; a schedule that was set
- * is used as it is. */
+ * is used as it is.  Single products (not the plans that a batch or a hierarchy
+ * replays) also forward the rows of unstructured operators without merging
+ * R*A first where the sample shows that merging saves little. */
 int sp3mm_set_tuning(const sp3mm_tuning *t);
 /* Autotuner: times the direct product R*A*P (opts->precision as in sp3mm_rap)
  * under candidate schedules, `reps` products each, and installs the fastest

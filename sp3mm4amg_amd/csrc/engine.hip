@@ -2015,15 +2015,11 @@ struct FusedPlan : PlanInput {
     // populations and offsets of build() hold, so only the values are
     // recomputed, straight into the output.  Binning, scan, gather and the
     // check of the sizes are left out (8 launches of 5 us and 24 us of gather
-    // for the finest product of a 96^3 hierarchy).  Not for plans with retried,
-    // spilled or scattered rows, which need their lists and slots.  The caller
-    // clears the error word.
-    bool fixed_ok() const
-    {
-        bool plain = built && !mixed && !f32 && nretry == 0 && nspill == 0 && !(lscatter && nlong > 0);
-        for (int i = 0; i < thr.nb; i++) plain = plain && !(cnt[i] > 0 && cfg[i].scatter);
-        return plain;
-    }
+    // for the finest product of a 96^3 hierarchy).  Not for plans with retried
+    // or spilled rows, which need their lists and slots (rows forwarded
+    // unmerged are in no plan that is replayed).  The caller clears the error
+    // word.
+    bool fixed_ok() const { return built && !mixed && !f32 && nretry == 0 && nspill == 0; }
     void record_fixed(Context *c, hipStream_t s)
     {
         for (int i = 0; i < thr.nb; i++)
