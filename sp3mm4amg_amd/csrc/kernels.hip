@@ -433,14 +433,18 @@ __device__ __forceinline__ void merge_plan(const int *raw, int nb, MergeRule rul
         dest[b] = b;
         start[b] = 0;
     }
+    // the bin folded into last, and the smallest bin whose rows came there under
+    // the rule for near bins
+    int last = -1, first = 0;
     for (int b = 0; b < nb; b++) {
         if (cnt[b] == 0 || cnt[b] > max(rule.any, rule.near)) continue;
-        int to = b + 1, low = b;  // low: the smallest bin whose rows are here
+        int to = b + 1;
         while (to < nb && cnt[to] == 0) to++;
         if (to >= nb) continue;
-        for (int c = b; c >= 0; c--)
-            if (dest[c] == b && raw[c] > 0) low = c;
+        const int low = b == last ? first : b;
         if (cnt[b] > rule.any && to - low > kMergeNear) continue;
+        last = to;
+        first = cnt[b] > rule.any ? low : to;
         for (int c = 0; c <= b; c++)
             if (dest[c] == b) {
                 dest[c] = to;

@@ -59,7 +59,7 @@ struct OneBin {
 };
 // Bins that fold into the next larger non-empty one: those of at most `any` rows
 // whatever its bound, those of at most `near` rows if it is at most kMergeNear
-// bins (a factor of 4) above the smallest bin folded.  Folded rows take the
+// bins (a factor of 4) above the smallest one folded that way.  Folded rows take the
 // larger bin's slots and its groups: 6,000 rows of 7 products under 50 of 3,500
 // took 240 us folded and 165 apart.  near 0: none.
 constexpr int kMergeNear = 2;
