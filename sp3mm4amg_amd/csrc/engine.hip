@@ -3170,7 +3170,7 @@ struct Batch {
     // 1 offsets): written to pinned host memory behind every build and run, so
     // that a result needs no read-back to be allocated (20 results of a mixed
     // batch: 740 us with two copies and a blocking wait each)
-    bool ready = false;           // the plan is built, and bounds are its output's
+    bool ready = false;           // the last build or run succeeded, and bounds are its output's
     Buf ends;                     // the offsets' positions
     int64_t *bounds = nullptr, *bounds_dev = nullptr;
 
@@ -3485,8 +3485,6 @@ static int batch_refit(Context *c, Batch *b)
     b->plan = std::move(old);
     b->graph = g;
     b->exec = x;
-    b->export_bounds(c->stream);  // the old output's again
-    b->ready = hipStreamSynchronize(c->stream) == hipSuccess;
     set_error("%s", why);
     return -1;
 }
@@ -3509,6 +3507,8 @@ int batch_run(void *h, bool use_graph, double *ms)
     const int rc = b->plan.check(c);
     if (ms) *ms = tm.ms(e0, e1);
     if (rc && b->plan.sampled && batch_refit(c, b) == 0) return batch_run(h, use_graph, ms);
+    // the offsets of a run that failed can end beyond the output's arrays
+    b->ready = rc == 0;
     return rc;
 }
 
@@ -3523,7 +3523,7 @@ int batch_result(void *h, int i, sp3mm_dmat &out)
         return -1;
     }
     if (!b->ready) {
-        set_error("batch: its last rebuild failed, there are no results");
+        set_error("batch: its last run or rebuild failed, there are no results");
         return -1;
     }
     const sp3mm_dmat &C = b->plan.C;
