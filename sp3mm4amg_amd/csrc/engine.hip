@@ -3169,29 +3169,49 @@ struct Batch {
     // where each product's entries begin and end in the packed output (count +
     // 1 offsets): written to pinned host memory behind every build and run, so
     // that a result needs no read-back to be allocated (20 results of a mixed
-    // batch: 740 us with two copies and a blocking wait each)
+    // batch: 740 us with two copies and a blocking wait each).  Up to
+    // kSharedBounds offsets go through the context's host block and are copied
+    // out after the wait that ends a build or a run; more through pinned memory
+    // of the batch's own (45 us more to create one).
+    static constexpr size_t kBoundsOff = 2048, kSharedBounds = (4096 - kBoundsOff) / 8;
+    static_assert(sizeof(Ctl) <= kBoundsOff, "the control block's mirror lies before it");
     bool ready = false;           // the last build or run succeeded, and bounds are its output's
-    Buf ends;                     // the offsets' positions
-    int64_t *bounds = nullptr, *bounds_dev = nullptr;
+    std::vector<int64_t> at;      // the offsets' positions,
+    Buf ends;                     // and on the device
+    int64_t *own_bounds = nullptr, *bounds_dev = nullptr;
+    std::vector<int64_t> shared_bounds;
+    const int64_t *bounds() const { return own_bounds ? own_bounds : shared_bounds.data(); }
 
     ~Batch()
     {
-        if (bounds) (void)hipHostFree(bounds);
+        if (own_bounds) (void)hipHostFree(own_bounds);
     }
-    // false: results read their offsets back
-    bool alloc_bounds(hipStream_t s)
+    // without bounds_dev results read their offsets back
+    void alloc_bounds(Context *c)
     {
-        std::vector<int64_t> at(roff);
+        at = roff;
         at.push_back(roff.back() + M.back());
         ends = Buf(at.size() * 8);
-        if (!ends.p || hipHostMalloc((void **)&bounds, at.size() * 8, hipHostMallocMapped) != hipSuccess ||
-            hipHostGetDevicePointer((void **)&bounds_dev, bounds, 0) != hipSuccess ||
-            hipMemcpyAsync(ends.p, at.data(), at.size() * 8, hipMemcpyHostToDevice, s) != hipSuccess ||
-            hipStreamSynchronize(s) != hipSuccess) {
+        hipError_t e = ends.p ? hipSuccess : hipErrorOutOfMemory;
+        if (at.size() <= kSharedBounds && c->host_small_dev) {
+            shared_bounds.resize(at.size());
+            bounds_dev = reinterpret_cast<int64_t *>(c->host_small_dev) + kBoundsOff / 8;
+        } else if (e == hipSuccess) {
+            e = hipHostMalloc((void **)&own_bounds, at.size() * 8, hipHostMallocMapped);
+            if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&bounds_dev, own_bounds, 0);
+        }
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(ends.p, at.data(), at.size() * 8, hipMemcpyHostToDevice, c->stream);
+        if (e != hipSuccess) {
             (void)hipGetLastError();
             bounds_dev = nullptr;
         }
-        return bounds_dev != nullptr;
+    }
+    // behind a wait for the export
+    void take_bounds(const Context *c)
+    {
+        if (!shared_bounds.empty())
+            memcpy(shared_bounds.data(), c->host_small + kBoundsOff / 8, shared_bounds.size() * 8);
     }
     void export_bounds(hipStream_t s)
     {
@@ -3225,6 +3245,7 @@ static int batch_build(Context *c, Batch *b, bool graph)
     const int e2 = tm.mark();
     (void)hipEventSynchronize(tm.ev[e2]);
     b->ms_build = tm.ms(e1, e2);
+    b->take_bounds(c);
     b->ready = true;
     if (graph) {
         hipStream_t s = c->stream;
@@ -3346,7 +3367,7 @@ void *batch_create(int count, const sp3mm_dmat *R, const sp3mm_dmat *A, const sp
     b->ms_pack = tm.ms(e0, e1);
     b->prec = prec;
     b->guard = guard > 0 ? guard : 1e-2;
-    (void)b->alloc_bounds(c->stream);
+    b->alloc_bounds(c);
     if (batch_build(c, b, graph)) {
         b->plan.release_all();
         dmat_release(b->Rb);
@@ -3509,6 +3530,7 @@ int batch_run(void *h, bool use_graph, double *ms)
     if (rc && b->plan.sampled && batch_refit(c, b) == 0) return batch_run(h, use_graph, ms);
     // the offsets of a run that failed can end beyond the output's arrays
     b->ready = rc == 0;
+    b->take_bounds(c);
     return rc;
 }
 
@@ -3529,8 +3551,8 @@ int batch_result(void *h, int i, sp3mm_dmat &out)
     const sp3mm_dmat &C = b->plan.C;
     int64_t lo = 0, hi = 0;
     if (b->bounds_dev) {
-        lo = b->bounds[i];
-        hi = b->bounds[i + 1];
+        lo = b->bounds()[i];
+        hi = b->bounds()[i + 1];
     } else {
         SP3MM_HIP(hipMemcpy(&lo, C.rp + b->roff[i], 8, hipMemcpyDeviceToHost));
         SP3MM_HIP(hipMemcpy(&hi, C.rp + b->roff[i] + b->M[i], 8, hipMemcpyDeviceToHost));

@@ -1,4 +1,5 @@
-"""Results of a batch: none after a run that failed."""
+"""Results of a batch: none after a run that failed, and each batch's own when
+runs of several batches alternate."""
 import numpy as np
 import pytest
 
@@ -41,3 +42,25 @@ def test_no_result_of_a_failed_run(graph):
             b.repack(As=[d[1]])
     finally:
         b.free()
+
+
+@pytest.mark.parametrize("counts", [(3, 2), (255, 1), (256, 254)])
+def test_alternating_batches(counts):
+    """Up to 255 products' entry ranges pass through memory that all batches
+    share, more through a batch's own."""
+    L.set_tuning(None)
+    rng = np.random.default_rng(2)
+    kinds = [[problems.poisson2d_sa(n)[k] for k in "RAP"] for n in (8, 11, 16)]
+    probs = [[kinds[i] for i in rng.integers(0, 3, n)] for n in counts]
+    dev = {id(k): [L.DeviceCSR.upload(m) for m in k] for k in kinds}
+    bs = [L.Batch(*([dev[id(k)][j] for k in ps] for j in range(3)), graph=i == 0) for i, ps in enumerate(probs)]
+    try:
+        for order in ((0, 1), (1, 0), (0, 0)):
+            for i in order:
+                bs[i].run(graph=i == 0)
+            for i in (0, 1):
+                for k in sorted({0, len(probs[i]) // 2, len(probs[i]) - 1}):
+                    _check(bs[i].result(k).download(), probs[i][k])
+    finally:
+        for b in bs:
+            b.free()
