@@ -1196,8 +1196,8 @@ static void fused_bins(size_t max_lds, bool mixed, const Tuning &tu, BinThreshol
 }
 
 // Table slots for rows of at most n distinct keys in the sample: a table at
-// most 3/4 full.  (27-point 100^3 product, 343 keys: 512 slots; a full table
-// sends its row to the long-row kernels, and probing grows past 3/4.)
+// most 3/4 full.  (27-point 100^3 product, 343 keys: 512 slots; a row that
+// fills its table is run again, and probing grows past 3/4.)
 static int sampled_slots(int n)
 {
     int h = kSampleTab;
@@ -1547,9 +1547,8 @@ struct FusedPlan : PlanInput {
     // the bin's bound).  Smaller bins take the tables of the next larger such
     // bin (a few sampled rows miss a bin's maximum: with 256 slots for 27-point
     // boundary rows of up to 245 keys those 3464 rows ran 275 us), larger ones
-    // keep the bound.  A row
-    // that fills its tables all the same is redone by the long-row kernels,
-    // as under any schedule.  false: nothing usable was sampled.
+    // keep the bound.  A row that fills its tables all the same runs once more
+    // (run_again).  false: nothing usable was sampled.
     bool apply_sample(Context *c, const SampleOut &so)
     {
         std::vector<FusedCfg> f(cfg);

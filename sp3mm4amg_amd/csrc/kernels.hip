@@ -878,7 +878,7 @@ __global__ void __launch_bounds__(256) k_direct(SpOperand R, SpOperand A, SpOper
 // a row of another length is an error instead of a retry.  Per replay of a
 // 96^3 hierarchy that saves the gathers of its first two products, 24 + 10 us.
 // A variant of its own: the same test at run time spills ten more scalar
-// registers, and a 27-point 64^3 mixed-input product took 669 instead of 595 us.
+// registers, and a 27-point 100^3 product with FP32 inputs took 669 instead of 595 us.
 template <int G, int U1, int U2, typename VT = double, bool PLACE = false>
 __global__ void __launch_bounds__(256, 6) k_direct_fused(SpOperand R, SpOperand A, SpOperand P,
                                                        const int32_t *__restrict__ rows,
@@ -2990,8 +2990,10 @@ void launch_window_direct(bool num, int blocks, size_t lds, const SpOperand &R, 
 // lanes alike; sub-groups of 16 lanes per row of P, as the other kernels use,
 // waited for the longest row between barriers (7.6 against 3.6 ms on the
 // 60,000-row lognormal operator, 1.3e9 products), four consecutive products
-// per lane tripled the L2 requests (6.0 ms).  Bound by the reads of P through
-// L2 (12 bytes per product of rows spread over 15 MB); kScatU = 2, 4, 8:
+// per lane tripled the L2 requests (6.0 ms).  Bound by the reads of P (12 bytes
+// per product of rows spread over 15 MB): 57% of the L2 requests miss, and 4.4
+// TB/s come from memory, a large copy's rate; LDS is active in 56% of the cycles.
+// kScatU = 2, 4, 8:
 // 4.24, 4.02, 3.96 ms per product, 100,000 rows 11.8, 10.4, 9.9.  The sums go into dense FP64 accumulators and
 // presence bits over all of P's columns; reading the bits in order emits the
 // sorted row into its slot of `cap` entries and clears the accumulators.

@@ -309,9 +309,9 @@ void launch_sa_rows(bool fill, const int64_t *rp, const int32_t *col, const doub
                     double *pval, int *maxlen, int longest, int *err, hipStream_t st);
 void launch_spmv(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz, const double *x,
                  const double *z, double *y, double alpha, double beta, hipStream_t st);
-// all sweeps in one launch over several workgroups, or in one workgroup when
-// the system fits in max_lds bytes of LDS (return false, launching nothing,
-// otherwise)
+// all sweeps in launches over several workgroups, which `cus` CUs must hold
+// together, or in one workgroup when the system fits in max_lds bytes of LDS
+// (return false, launching nothing, otherwise)
 bool launch_jacobi_grid(const int64_t *rp, const int32_t *col, const double *val, int64_t M, int64_t nnz,
                         const double *b, double *x, void *buf, double omega, int sweeps, bool from_zero, int *err,
                         int cus, hipStream_t st);
