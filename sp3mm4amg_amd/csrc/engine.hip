@@ -1216,10 +1216,7 @@ static int likely_bin(const BinThresholds &thr, const sp3mm_dmat &R, const sp3mm
     return b >= thr.nb ? -1 : b;
 }
 
-// FusedPlan: the one-pass direct pipeline.  build() runs it eagerly, reading
-// counters back to size bins, scratch slots and the output; record() enqueues
-// the same kernels for the sizes found by build() with no host
-// synchronisation, so it can be captured into a HIP graph and replayed.
+// What a FusedPlan is built from.
 struct PlanInput {
     sp3mm_dmat R{}, A{}, P{};
     bool mixed = false;  // FP32-pair accumulation kernel
@@ -1240,6 +1237,11 @@ struct PlanInput {
     // R*(A*P) as two SpGEMMs; see wants_reassoc)
     bool reassoc_ok = false;
 };
+
+// FusedPlan: the one-pass direct pipeline.  build() runs it eagerly, reading
+// counters back to size bins, scratch slots and the output; record() enqueues
+// the same kernels for the sizes found by build() with no host
+// synchronisation, so it can be captured into a HIP graph and replayed.
 struct FusedPlan : PlanInput {
     BinThresholds thr{};
     std::vector<FusedCfg> cfg;
@@ -1592,7 +1594,8 @@ struct FusedPlan : PlanInput {
     // holds both (one of 64 slots for 60 keys took 97 us for 133 rows).  40,000
     // rows of 20 x 9 products, 133 of them scattered over 160,000 columns, which
     // the long-row kernels take one by one in HBM: 143 us unsampled, 340 when
-    // the sample missed the 133, 224 this way.
+    // the sample missed the 133, 224 this way.  All but the 64 sampled of 60,000
+    // rows missed: 5.0 ms and 1.2 (a batch's replays 4.4 and 0.22).
     void run_again(Context *c, hipStream_t s)
     {
         int b = thr.nb - 1;
@@ -1600,9 +1603,10 @@ struct FusedPlan : PlanInput {
         FusedCfg f = unsampled[b];
         f.G = f.H1 <= 512 ? 64 : 256;
         const int least = std::max(f.H2, f.G);
-        for (f.H2 = std::max(f.H1, f.G); f.H2 > least && fused_lds(f.G, f.H1, f.H2) > c->max_lds; f.H2 /= 2) {
-        }
-        if (fused_lds(f.G, f.H1, f.H2) > c->max_lds) return;
+        f.H2 = std::max(f.H1, f.G);
+        auto slots = [&] { return (size_t)nretry * f.H2 * 12; };
+        while (f.H2 > least && (fused_lds(f.G, f.H1, f.H2) > c->max_lds || slots() > ((size_t)1 << 30))) f.H2 /= 2;
+        if (fused_lds(f.G, f.H1, f.H2) > c->max_lds || slots() > ((size_t)4 << 30)) return;
         Buf list((size_t)nretry * 4);
         aslotn = Buf((size_t)nretry * 4);
         acol = Buf((size_t)nretry * f.H2 * 4);
@@ -2051,20 +2055,29 @@ struct FusedPlan : PlanInput {
 // plan.build().  Slots for sampled tables, and the dense ones of unmerged rows
 // (up to 4 GiB), can take memory that the schedule's own tables do without: an
 // adapted plan that fails is built once more as its schedule stands.  So is one
-// to be replayed with rows that its sampled tables do not hold: every replay
-// would run them on the long-row kernels.
+// to be replayed with rows that its sampled tables do not hold (every replay
+// would run them on the long-row kernels), if there is room for a second plan.
 static int build_plan(Context *c, FusedPlan &plan, Timer &tm)
 {
     PlanInput in = plan;
-    const int rc = plan.build(c, tm);
-    if (rc == 0 && !(plan.keep && plan.sampled && plan.nretry > 0)) return 0;
+    const bool built = plan.build(c, tm) == 0;
+    if (built && !(plan.keep && plan.sampled && plan.nretry > 0)) return 0;
     if (!in.adapt) return -1;
-    plan.release_all();
+    FusedPlan adapted;
+    if (built) adapted = std::move(plan);
+    else plan.release_all();
     plan = FusedPlan();
     in.adapt = false;
     static_cast<PlanInput &>(plan) = in;
     clear_error();
-    return plan.build(c, tm);
+    int rc = plan.build(c, tm);
+    if (rc && built) {
+        std::swap(plan, adapted);
+        clear_error();
+        rc = 0;
+    }
+    if (built) adapted.release_all();
+    return rc;
 }
 
 static int rap_direct_fused(const sp3mm_dmat &R, const sp3mm_dmat &A, const sp3mm_dmat &P, sp3mm_dmat &C,

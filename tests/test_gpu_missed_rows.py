@@ -37,6 +37,41 @@ def test_one_off_product(nout, per_row, outliers, left, f32):
     assert st["guarded_entries"] == left
 
 
+def _sampled_rows(m):
+    """The rows of R that the library samples: one per 64th, at a pseudo-random place in it."""
+    u = (1 << 64) - 1
+    rows = []
+    for p in range(64):
+        z = 0x9E3779B97F4A7C15 * (p + 2) & u
+        z = (z ^ z >> 30) * 0xBF58476D1CE4E5B9 & u
+        z = (z ^ z >> 27) * 0x94D049BB133111EB & u
+        lo, hi = p * m // 64, (p + 1) * m // 64
+        rows.append(min(lo + ((z >> 32 | 1) * max(1, hi - lo) >> 32), m - 1))
+    return rows
+
+
+@pytest.mark.parametrize("graph", [None, False, True])
+def test_every_row_but_the_sampled_ones(graph):
+    L.set_tuning(None)
+    m = 60_000
+    ops = _clustered(m, np.setdiff1d(np.arange(m), _sampled_rows(m)))
+    want = O.sp3mm_merged(*ops)
+    d = [L.DeviceCSR.upload(x) for x in ops]
+    if graph is None:
+        out, st = L.rap(*d)
+        print(f"{st['ms_total']:.3f} ms, {st['guarded_entries']} rows on the long-row kernels")
+        _check(out.download(), want)
+        assert st["guarded_entries"] == 0
+        return
+    b = L.Batch(*([x] for x in d), graph=graph)
+    try:
+        for _ in range(2):
+            print(f"{b.run(graph=graph):.3f} ms")
+            _check(b.result(0).download(), want)
+    finally:
+        b.free()
+
+
 def test_rows_of_several_bins():
     """Short rows (a bound of 24) beside the clustered ones: the missed rows of
     both bins run in the larger bin's tables."""
